@@ -130,16 +130,19 @@ __device__ __forceinline__ int take_ticket(int* ctr) {
 }
 
 // nblocks: workgroups that take tickets from ctr (the whole grid unless a
-// launch splits its workgroups over several ticket counters).
-__device__ __forceinline__ void retire_ticket(int* ctr, int nblocks = -1) {
+// launch splits its workgroups over several ticket counters).  True in thread
+// 0 of the last one.
+__device__ __forceinline__ bool retire_ticket(int* ctr, int nblocks = -1) {
     __syncthreads();
     if (threadIdx.x == 0) {
         int done = __hip_atomic_fetch_add(&ctr[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (done == (nblocks < 0 ? static_cast<int>(gridDim.x) : nblocks) - 1) {
             __hip_atomic_store(&ctr[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&ctr[1], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return true;
         }
     }
+    return false;
 }
 
 // v of the lane K places up within the lane's row of 16 (DPP row shift; 0

@@ -58,6 +58,23 @@ struct SweepPack {
     int max_np = 0;                 // most PassDesc records of one block
     int pass_g = 0;                 // lanes per row the pass list was built for
 };
+// Chunk stream of one direction (ilu_stream.hip), built for a partition and a
+// lanes-per-row count; lds == 0 after a build that did not fit the LDS.
+struct SweepStream {
+    DevBuf<int> kptr, cptr;         // per processed block: first schedule position, first chunk
+    DevBuf<int> irange;             // per processed block: (first mailbox word, count) of its imports
+    DevBuf<uint64_t> mail;          // mailboxes, two generations of mail_words
+    DevBuf<int> gen;                // generation of the next launch
+    DevBuf<int> scol, ssrc;         // per lane: (LDS slots, byte offset of its result); factor entry (-1: none)
+    DevBuf<int> srow;               // per chunk row: row or -1
+    DevBuf<double> sval64, sdiag;   // per lane values; per chunk row (u_ii, 1 / u_ii)
+    DevBuf<float> sval32;
+    long nchunk = 0, mail_words = 0;
+    int max_chunks = 0;             // most chunks of one block
+    size_t lds = 0;
+    int version = -1, g = 0;        // partition and lanes per row it was built for
+    long factors = -1;              // factorization its values were gathered from
+};
 // Record streams of the wave-specialised sweep (mode 5) for one direction,
 // built for a partition and a lanes-per-row count.
 struct WsPack {
@@ -133,6 +150,7 @@ struct lljbash::IluSolver::Ext {
     // block sweep over record streams (k_sweep_ws).
     int mode_l = 0, mode_u = 0;
     pilu::SweepPack pack_l, pack_u;
+    pilu::SweepStream stream_l, stream_u;
     pilu::WsPack ws_l, ws_u;
     // Block partition of the rows: contiguous blocks of blk_rows rows, or
     // tiles of the grid (tile[] != 0, grid[] declared by SetGridShape).

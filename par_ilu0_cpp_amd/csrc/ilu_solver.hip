@@ -24,6 +24,7 @@
 
 #include "ilu_internal.hpp"
 #include "ilu_kernels.hpp"
+#include "ilu_stream.hpp"
 #include "ilu_sweep_ws.hpp"
 #include "iluk_device.hpp"
 
@@ -1030,21 +1031,27 @@ void gather_pack(Ext* e, SweepPack& pk, bool upper) {
     pk.factors = e->factor_version;
 }
 
-void ensure_packs(Ext* e) {
+void ensure_pack(Ext* e, bool upper) {
     if (e->nblk <= 0) throw std::runtime_error("packed sweep needs a block partition");
     PhaseTimer pt("packs", e->stream);
-    if (e->pack_l.version != e->part_version) {
-        build_pack(e, false, e->pack_l);
-        pt.mark("L pack");
+    SweepPack& pk = upper ? e->pack_u : e->pack_l;
+    if (pk.version != e->part_version) {
+        build_pack(e, upper, pk);
+        pt.mark(upper ? "U pack" : "L pack");
     }
-    if (e->pack_u.version != e->part_version) {
-        build_pack(e, true, e->pack_u);
-        pt.mark("U pack");
-    }
-    if (e->factored) {
-        if (e->pack_l.factors != e->factor_version) gather_pack(e, e->pack_l, false);
-        if (e->pack_u.factors != e->factor_version) gather_pack(e, e->pack_u, true);
-    }
+    if (e->factored && pk.factors != e->factor_version) gather_pack(e, pk, upper);
+}
+
+int pp_lanes(int lanes);
+
+// What modes 2 and 3 of one direction sweep over for a configured lane
+// count: the chunk stream where a row's entries fit its lanes and a block
+// its LDS, else the packed factors and their pass list.
+void ensure_packed(Ext* e, bool upper, int lanes) {
+    const int g = pp_lanes(lanes);
+    if (ensure_stream(e, upper, g)) return;
+    ensure_pack(e, upper);
+    build_passes(e, upper ? e->pack_u : e->pack_l, g);
 }
 
 // ---------------------------------------------------------------------
@@ -1453,12 +1460,11 @@ int pp_lanes(int lanes) { return lanes == 1 || lanes == 2 || lanes == 4 || lanes
 void prepare_modes(Ext* e) {
     const bool pp_l = e->mode_l >= 2 && e->mode_l <= 3, pp_u = e->mode_u >= 2 && e->mode_u <= 3;
     if (pp_l || pp_u) {
-        ensure_packs(e);
-        // pass lists for the lanes the packed sweeps will run with
+        // for the lanes the packed sweeps will run with
         PhaseTimer pt("packs", e->stream);
-        if (pp_l) build_passes(e, e->pack_l, pp_lanes(effective_lanes(e, false)));
-        if (pp_u) build_passes(e, e->pack_u, pp_lanes(effective_lanes(e, true)));
-        pt.mark("pass lists");
+        if (pp_l) ensure_packed(e, false, effective_lanes(e, false));
+        if (pp_u) ensure_packed(e, true, effective_lanes(e, true));
+        pt.mark("streams or pass lists");
     }
     if (e->mode_l == 5) ensure_ws(e, false, ws_lanes(effective_lanes(e, false)));
     if (e->mode_u == 5) ensure_ws(e, true, ws_lanes(effective_lanes(e, true)));
@@ -1525,10 +1531,11 @@ constexpr size_t kMaxLds = 160 * 1024;
 // True when the packed sweep with G lanes per row fits the LDS in both
 // directions for the current partition.
 bool pp_fits(Ext* e, int G) {
-    ensure_packs(e);
-    build_passes(e, e->pack_l, G);
-    build_passes(e, e->pack_u, G);
-    return pp_lds_bytes(e, e->pack_l) <= kMaxLds && pp_lds_bytes(e, e->pack_u) <= kMaxLds;
+    for (const bool upper : {false, true}) {
+        ensure_packed(e, upper, G);
+        if (!stream_applies(e, upper, G) && pp_lds_bytes(e, upper ? e->pack_u : e->pack_l) > kMaxLds) return false;
+    }
+    return true;
 }
 
 template <int G, int S, typename T, bool UPPER, bool FLAGS>
@@ -1671,7 +1678,11 @@ void sweep_dispatch(int lanes, Ext* e, const T* val, const double* b, double* ou
         return;
     }
     if (mode >= 2 && mode <= 3 && e->nblk > 0) {
-        ensure_packs(e);
+        if (ensure_stream(e, UPPER, pp_lanes(lanes))) {
+            sweep_stream(e, UPPER, b, out, reset, gate, ctr, e->err.get() + kErrSweep);
+            return;
+        }
+        ensure_pack(e, UPPER);
         sweep_pp_dispatch<T, UPPER>(lanes, e, b, out, reset, gate, ctr);
         return;
     }
@@ -1757,6 +1768,8 @@ bool run_factor(Ext* e) {
     ++e->factor_version;
     gather_pack(e, e->pack_l, false);
     gather_pack(e, e->pack_u, true);
+    gather_stream(e, false);
+    gather_stream(e, true);
     if (ws_current(e, e->ws_l, e->ws_l.g)) gather_ws(e, e->ws_l);
     if (ws_current(e, e->ws_u, e->ws_u.g)) gather_ws(e, e->ws_u);
     return (err & 1) == 0 && e->factor_status == 0;
@@ -1776,9 +1789,14 @@ void show_algorithm(const lljbash::IluSolver* solver) {
     if (v && *v && std::strcmp(v, "0") != 0) std::printf("%s\n", solver->DescribeSchedule().c_str());
 }
 
-// Sweep kinds whose output must hold kPending in every slot on entry
-// (value-flag synchronisation through the output vector).
-bool flags_in_output(int mode) { return mode >= 0 && mode <= 3; }
+// Whether the configured sweep of a direction synchronises through value-flags
+// in its output, which must then hold kPending in every slot on entry: modes
+// 0 to 3, unless a chunk stream takes the place of the packed factors.
+bool flags_in_output(Ext* e, bool upper) {
+    const int mode = upper ? e->mode_u : e->mode_l;
+    if (mode < 0 || mode > 3) return false;
+    return mode < 2 || e->nblk <= 0 || !ensure_stream(e, upper, pp_lanes(effective_lanes(e, upper)));
+}
 
 // The forward sweep b -> y, then the backward sweep y -> x.  Each sweep
 // re-arms the other one's output where the other one synchronises through
@@ -1790,8 +1808,8 @@ bool flags_in_output(int mode) { return mode >= 0 && mode <= 3; }
 void sweep_pair(Ext* e, const double* d_b, double* d_x, double* y, const int* gate, int* ctr, hipEvent_t* ev) {
     hipStream_t s = e->stream;
     const int gl = effective_lanes(e, false), gu = effective_lanes(e, true);
-    double* reset_l = flags_in_output(e->mode_u) ? d_x : nullptr;
-    double* reset_u = flags_in_output(e->mode_l) ? y : nullptr;
+    double* reset_l = flags_in_output(e, true) ? d_x : nullptr;
+    double* reset_u = flags_in_output(e, false) ? y : nullptr;
     if (ev) PILU_HIP(hipEventRecord(ev[0], s));
     if (e->precision == 32) sweep_dispatch<float, false>(gl, e, e->fac32.get(), d_b, y, reset_l, gate, ctr);
     else sweep_dispatch<double, false>(gl, e, e->fac.get(), d_b, y, reset_l, gate, ctr);
@@ -1805,7 +1823,7 @@ void sweep_pair(Ext* e, const double* d_b, double* d_x, double* y, const int* ga
 // Fills the solver's y with kPending when the forward sweep synchronises
 // through it and the last backward sweep did not re-arm it.
 void arm_y(Ext* e) {
-    if (flags_in_output(e->mode_l) && !e->y_armed)
+    if (flags_in_output(e, false) && !e->y_armed)
         k_fill_u64<<<grid_for(e->n, 256 * 8), 256, 0, e->stream>>>(e->n, reinterpret_cast<uint64_t*>(e->y.get()),
                                                                     kPending);
 }
@@ -1815,7 +1833,7 @@ void ilu_apply(Ext* e, const double* d_b, double* d_x, const int* gate) {
     if (!e->factored) throw std::runtime_error("IluSolver: Factorize has not been called");
     arm_y(e);
     sweep_pair(e, d_b, d_x, e->y.get(), gate, e->ctr.get() + 4, nullptr);
-    e->y_armed = flags_in_output(e->mode_l);
+    e->y_armed = flags_in_output(e, false);
 }
 
 __global__ void k_scale_vec(long n, double alpha, double* __restrict__ y) {
@@ -1838,7 +1856,7 @@ void ilu_trsv(Ext* e, bool upper, double alpha, const double* d_x, double* d_y) 
         in = e->y.get();
         e->y_armed = false;
     }
-    if (flags_in_output(upper ? e->mode_u : e->mode_l))
+    if (flags_in_output(e, upper))
         k_fill_u64<<<grid_for(e->n, 256 * 8), 256, 0, s>>>(e->n, reinterpret_cast<uint64_t*>(d_y), kPending);
     const int g = effective_lanes(e, upper);
     int* ctr = e->ctr.get() + (upper ? 6 : 4);
@@ -2108,7 +2126,7 @@ void time_sweeps(Ext* e, int lanes, const double* b, double* x, int reps, hipEve
     for (int r = 0; r < reps; ++r) {
         arm_y(e);
         sweep_pair(e, b, x, e->y.get(), nullptr, e->ctr.get() + 4, ev);
-        e->y_armed = flags_in_output(e->mode_l);
+        e->y_armed = flags_in_output(e, false);
         PILU_HIP(hipEventSynchronize(ev[2]));
         float a = 0.f, c = 0.f;
         PILU_HIP(hipEventElapsedTime(&a, ev[0], ev[1]));
@@ -2315,11 +2333,21 @@ std::string IluSolver::DescribeSchedule() const {
                   e->max_block_rows, e->mode_l,
                   pilu::effective_lanes(e, false), e->mode_u, pilu::effective_lanes(e, true));
     std::string js(buf);
-    const bool live_l = e->nblk > 0 && e->pack_l.version == e->part_version;
-    const bool live_u = e->nblk > 0 && e->pack_u.version == e->part_version;
+    // a direction's chunk stream takes the place of its pack
+    auto packed = [&](const pilu::SweepPack& pk, const pilu::SweepStream& st, int max_w) {
+        if (e->nblk > 0 && st.version == e->part_version && st.lds > 0) {
+            char b[256];
+            std::snprintf(b, sizeof(b),
+                          "{\"entries\": %ld, \"max_width\": %d, \"lanes\": %d, \"max_passes_per_block\": %d, "
+                          "\"lds_bytes\": %zu}",
+                          st.nchunk * 64, max_w, st.g, st.max_chunks, st.lds);
+            return std::string(b);
+        }
+        return e->nblk > 0 && pk.version == e->part_version ? pack(pk) : std::string("null");
+    };
     js += "\"lv_cached_levels\": [" + std::to_string(e->lvcached_l) + ", " + std::to_string(e->lvcached_u) + "], ";
-    js += "\"pack_l\": " + (live_l ? pack(e->pack_l) : std::string("null"));
-    js += ", \"pack_u\": " + (live_u ? pack(e->pack_u) : std::string("null"));
+    js += "\"pack_l\": " + packed(e->pack_l, e->stream_l, e->max_lo);
+    js += ", \"pack_u\": " + packed(e->pack_u, e->stream_u, e->max_up);
     // wave-specialised streams: LDS per workgroup and how many fit a CU's 160 KiB
     auto ws = [&](const pilu::WsPack& wp) {
         if (wp.version != e->part_version || !wp.stream.get()) return std::string("null");
