@@ -70,9 +70,9 @@ struct SweepStream {
     DevBuf<double> sval64, sdiag;   // per lane values; per chunk row (u_ii, 1 / u_ii)
     DevBuf<float> sval32;
     long nchunk = 0, mail_words = 0;
-    int max_chunks = 0;             // most chunks of one block
+    int nblk = 0, max_chunks = 0;   // blocks; most chunks of one block
     size_t lds = 0;
-    int version = -1, g = 0;        // partition and lanes per row it was built for
+    int version = -1, g = 0;        // partition (default streams: pattern) and lanes per row it was built for
     long factors = -1;              // factorization its values were gathered from
 };
 // Record streams of the wave-specialised sweep (mode 5) for one direction,
@@ -151,6 +151,13 @@ struct lljbash::IluSolver::Ext {
     int mode_l = 0, mode_u = 0;
     pilu::SweepPack pack_l, pack_u;
     pilu::SweepStream stream_l, stream_u;
+    // Sweeps of a solver whose sweep shape was never set (sweep_default):
+    // level-scheduled rows at first, chunk streams after a few applies where
+    // the pattern suits them (auto_l / auto_u, decided for auto_pattern and
+    // the lanes).
+    bool sweep_default = true, auto_on = false;
+    int auto_applies = 0, auto_pattern = -1, auto_lanes[2] = {0, 0};
+    pilu::SweepStream auto_l, auto_u;
     pilu::WsPack ws_l, ws_u;
     // Block partition of the rows: contiguous blocks of blk_rows rows, or
     // tiles of the grid (tile[] != 0, grid[] declared by SetGridShape).

@@ -807,6 +807,10 @@ void analyse(Ext* e) {
     e->tile[0] = e->tile[1] = e->tile[2] = 0;
     e->grid[0] = e->grid[1] = e->grid[2] = 0;
     ++e->part_version;
+    e->sweep_default = true;
+    e->auto_on = false;
+    e->auto_applies = 0;
+    e->auto_pattern = -1;
     e->analysed = true;
 }
 
@@ -1043,13 +1047,31 @@ void ensure_pack(Ext* e, bool upper) {
 }
 
 int pp_lanes(int lanes);
+int effective_lanes(const Ext* e, bool upper);
+
+// The current partition's chunk stream of one direction for G lanes per row,
+// built and filled where it is missing or stale; null where the packed
+// factors have to be swept.
+const SweepStream* packed_stream(Ext* e, bool upper, int G) {
+    SweepStream& st = upper ? e->stream_u : e->stream_l;
+    if (e->nblk <= 0 || !stream_width_fits(e, upper, G)) return nullptr;
+    if (st.version != e->part_version || st.g != G) {
+        const StreamSchedule sc{(upper ? e->bperm_u : e->bperm_l).get(), (upper ? e->blev_u : e->blev_l).get(),
+                                (upper ? e->loff_u : e->loff_l).get(), e->block_of.get(), e->nblk};
+        build_stream(e, upper, G, sc, st);
+        st.version = e->part_version;
+    }
+    if (st.lds == 0) return nullptr;
+    if (e->factored && st.factors != e->factor_version) gather_stream(e, upper, st);
+    return &st;
+}
 
 // What modes 2 and 3 of one direction sweep over for a configured lane
 // count: the chunk stream where a row's entries fit its lanes and a block
 // its LDS, else the packed factors and their pass list.
 void ensure_packed(Ext* e, bool upper, int lanes) {
     const int g = pp_lanes(lanes);
-    if (ensure_stream(e, upper, g)) return;
+    if (packed_stream(e, upper, g)) return;
     ensure_pack(e, upper);
     build_passes(e, upper ? e->pack_u : e->pack_l, g);
 }
@@ -1445,7 +1467,7 @@ void sweep_ws_one(Ext* e, const double* b, double* out, double* reset, const int
     if (other_ws) other.face_armed = true;
 }
 
-int effective_lanes(const Ext* e, bool upper);
+
 
 // Lanes per row of the wave-specialised sweep: the configured count, at
 // most 16 (records hold 64 / G rows).
@@ -1533,7 +1555,7 @@ constexpr size_t kMaxLds = 160 * 1024;
 bool pp_fits(Ext* e, int G) {
     for (const bool upper : {false, true}) {
         ensure_packed(e, upper, G);
-        if (!stream_applies(e, upper, G) && pp_lds_bytes(e, upper ? e->pack_u : e->pack_l) > kMaxLds) return false;
+        if (!packed_stream(e, upper, G) && pp_lds_bytes(e, upper ? e->pack_u : e->pack_l) > kMaxLds) return false;
     }
     return true;
 }
@@ -1657,6 +1679,171 @@ void sweep_lv_one(Ext* e, const T* val, const double* b, double* out, double* re
                                                  watchdog_ticks(e->watchdog_s), cached > 0 ? 1 : 0);
 }
 
+// ---------------------------------------------------------------------
+// Sweeps of a solver whose sweep shape was never set.  Level-scheduled rows
+// need no more than the analysis, but pay a hand-off through memory per
+// level (1.05 us at 2D Poisson 64^2, 1.85 us at 77 x 59 x 91 ILU(1)).  Once a
+// pattern has been applied kAutoAfter times they are replaced by chunk
+// streams where rows are short and
+//   * the whole matrix fits one workgroup's LDS, or
+//   * the pattern is that of a grid, whose shape the offsets of its entries
+//     give away; the tiles then come from use_tiles, which derives their
+//     skew from the pattern, so a wrong guess costs time but never a result.
+// Every sum keeps its order: results do not change.
+// ---------------------------------------------------------------------
+constexpr int kAutoAfter = 2;
+
+// Distinct positive offsets row - column of L's entries in tab (0: free);
+// *over is set when there are more than kOffsets.
+constexpr int kOffsets = 16;
+__global__ void k_offsets(int n, const int* __restrict__ rp, const int* __restrict__ dg, const int* __restrict__ ci,
+                          int* tab, int* over) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    for (int p = rp[i]; p < dg[i]; ++p) {
+        const int d = i - ci[p];
+        int k = 0;
+        for (; k < kOffsets; ++k) {
+            int v = peek_int(tab + k);
+            if (v == 0) v = atomicCAS(tab + k, 0, d);
+            if (v == 0 || v == d) break;
+        }
+        if (k == kOffsets) *over = 1;
+    }
+}
+
+// Shape of the natural-order grid whose neighbour offsets are `d` (sorted):
+// the nx and nx * ny among them (or n, for one plane) that divide n and give
+// every offset at most two steps per axis, in the fewest steps in all.
+bool infer_grid(int n, const std::vector<int>& d, int* shape) {
+    if (d.empty() || d[0] != 1) return false;
+    long best = LONG_MAX;
+    std::vector<int> planes = d;
+    planes.push_back(n);
+    for (const long nx : d)
+        for (const long nxy : planes) {
+            if (nx < 2 || nxy <= nx || nxy % nx || n % nxy) continue;
+            long steps = 0;
+            bool ok = true;
+            for (const long v : d) {
+                const long z = (v + nxy / 2) / nxy, r = v - z * nxy;
+                const long y = (r >= 0 ? r + nx / 2 : r - nx / 2) / nx, x = r - y * nx;
+                ok = ok && z <= 2 && std::abs(y) <= 2 && std::abs(x) <= 2 && (nxy < n || z == 0);
+                steps += z + std::abs(y) + std::abs(x);
+            }
+            if (ok && steps < best) {
+                best = steps;
+                shape[0] = static_cast<int>(nx);
+                shape[1] = static_cast<int>(nxy / nx);
+                shape[2] = static_cast<int>(n / nxy);
+            }
+        }
+    return best < LONG_MAX;
+}
+
+// One workgroup walks a level in about 0.16 us plus 0.2 us per 8 chunks (64 / G
+// rows each); tiles share wide levels out but pay a hand-off of 1 to 2 us per
+// tile on the way.  Measured per L+U apply, one workgroup against tiles: 2D
+// Poisson 64^2 (2 chunks per level) 49 and 50 us, 128^2 (4) 112 and 91 us,
+// 12^3 ILU(1) (3) 34 and 47 us, 20^3 ILU(1) (9) 97 and 69 us, 25^3 ILU(0) (13)
+// 93 and 51 us; level-scheduled rows took 265, 568, 143, 280 and 201 us.  So
+// one workgroup up to kAutoNarrow chunks per level, tiles of a grid beyond
+// that, and without a grid one workgroup up to kAutoWide (a level-scheduled
+// level is about 1 us).
+constexpr int kAutoNarrow = 4, kAutoWide = 40;
+
+bool build_auto(Ext* e) {
+    const int gl = effective_lanes(e, false), gu = effective_lanes(e, true);
+    if (!stream_width_fits(e, false, gl) || !stream_width_fits(e, true, gu)) return false;
+    const int n = e->n;
+    hipStream_t s = e->stream;
+    const long level_rows = static_cast<long>(64 / std::max(gl, gu)) * std::min(e->nlev_l, e->nlev_u);
+    auto one_block = [&]() {
+        DevBuf<int> block_of(n), blev(4);
+        const int hb[4] = {0, e->nlev_l, 0, e->nlev_u};
+        PILU_HIP(hipMemcpyAsync(blev.get(), hb, sizeof(hb), hipMemcpyHostToDevice, s));
+        k_fill_int<<<grid_for(n, 256 * 8), 256, 0, s>>>(n, block_of.get(), 0);
+        return build_stream(e, false, gl, {e->perm_l.get(), blev.get(), e->lvoff_l.get(), block_of.get(), 1}, e->auto_l) &&
+               build_stream(e, true, gu, {e->perm_u.get(), blev.get() + 2, e->lvoff_u.get(), block_of.get(), 1}, e->auto_u);
+    };
+    if (n <= kMaxBlockRows && n <= kAutoNarrow * level_rows) return one_block();
+    DevBuf<int> tab(kOffsets + 1);
+    k_fill_int<<<1, 64, 0, s>>>(kOffsets + 1, tab.get(), 0);
+    k_offsets<<<grid_for(n, 256), 256, 0, s>>>(n, e->rp.get(), e->dg.get(), e->ci.get(), tab.get(), tab.get() + kOffsets);
+    PILU_HIP(hipGetLastError());
+    int h[kOffsets + 1];
+    PILU_HIP(hipMemcpyAsync(h, tab.get(), sizeof(h), hipMemcpyDeviceToHost, s));
+    PILU_HIP(hipStreamSynchronize(s));
+    std::vector<int> d;
+    for (int k = 0; k < kOffsets; ++k)
+        if (h[k] != 0) d.push_back(h[k]);
+    std::sort(d.begin(), d.end());
+    int shape[3];
+    if (h[kOffsets] || !infer_grid(n, d, shape))
+        return n <= kMaxBlockRows && n <= kAutoWide * level_rows && one_block();
+    // the partition is only needed for the build: what describes a configured
+    // one is put back
+    struct Restore {
+        Ext* e;
+        int grid[3], tile[3], skew[3], blk, nblk, rows;
+        explicit Restore(Ext* x) : e(x), blk(x->blk_rows), nblk(x->nblk), rows(x->max_block_rows) {
+            std::copy(x->grid, x->grid + 3, grid);
+            std::copy(x->tile, x->tile + 3, tile);
+            std::copy(x->skew, x->skew + 3, skew);
+        }
+        ~Restore() {
+            std::copy(grid, grid + 3, e->grid);
+            std::copy(tile, tile + 3, e->tile);
+            std::copy(skew, skew + 3, e->skew);
+            e->blk_rows = blk;
+            e->nblk = nblk;
+            e->max_block_rows = rows;
+            for (auto* b : {&e->block_of, &e->bperm_l, &e->bperm_u, &e->blev_l, &e->blev_u, &e->loff_l, &e->loff_u})
+                b->release();
+        }
+    } restore(e);
+    std::copy(shape, shape + 3, e->grid);
+    // 128 x 8 x 4 is within 4% of the fastest shape at 112^3 ILU(1) (474 us
+    // against 457 for 128 x 4 x 4) and the fastest at 77 x 59 x 91 (286, 305)
+    // and at 128^3 ILU(0) (310, 349); 256 x 32 in 2D (512 x 400 ILU(1): 413 us,
+    // 425 for 128 x 32)
+    if (shape[2] == 1) use_tiles(e, std::min(shape[0], 256), 32, 1);
+    else use_tiles(e, std::min(shape[0], 128), 8, 4);
+    return build_stream(e, false, gl, {e->bperm_l.get(), e->blev_l.get(), e->loff_l.get(), e->block_of.get(), e->nblk}, e->auto_l) &&
+           build_stream(e, true, gu, {e->bperm_u.get(), e->blev_u.get(), e->loff_u.get(), e->block_of.get(), e->nblk}, e->auto_u);
+}
+
+// Counts an apply of a default-shaped solver and decides once per pattern
+// and lane count.
+void count_default_apply(Ext* e) {
+    if (!e->sweep_default || e->mode_l != 0 || e->mode_u != 0) return;
+    const int gl = effective_lanes(e, false), gu = effective_lanes(e, true);
+    if (e->auto_pattern == e->pattern_version && e->auto_lanes[0] == gl && e->auto_lanes[1] == gu) return;
+    if (e->auto_applies++ < kAutoAfter) return;
+    SetupScope scope(e->stream);
+    e->auto_on = false;
+    e->auto_pattern = e->pattern_version;
+    e->auto_lanes[0] = gl;
+    e->auto_lanes[1] = gu;
+    try {
+        e->auto_on = build_auto(e);
+    } catch (const std::runtime_error&) {
+        // no acyclic tiles, or no memory for the streams: level-scheduled rows stay
+        (void)hipGetLastError();
+    }
+    e->auto_l.version = e->auto_u.version = e->auto_on ? e->pattern_version : -1;
+}
+
+// The stream that replaces the level-scheduled sweep of a direction, or null.
+const SweepStream* auto_stream(Ext* e, bool upper) {
+    SweepStream& st = upper ? e->auto_u : e->auto_l;
+    if (!e->sweep_default || !e->auto_on || st.version != e->pattern_version ||
+        st.g != effective_lanes(e, upper))
+        return nullptr;
+    if (e->factored && st.factors != e->factor_version) gather_stream(e, upper, st);
+    return &st;
+}
+
 template <typename T, bool UPPER>
 void sweep_dispatch(int lanes, Ext* e, const T* val, const double* b, double* out, double* reset,
                     const int* gate, int* ctr) {
@@ -1678,8 +1865,8 @@ void sweep_dispatch(int lanes, Ext* e, const T* val, const double* b, double* ou
         return;
     }
     if (mode >= 2 && mode <= 3 && e->nblk > 0) {
-        if (ensure_stream(e, UPPER, pp_lanes(lanes))) {
-            sweep_stream(e, UPPER, b, out, reset, gate, ctr, e->err.get() + kErrSweep);
+        if (const SweepStream* st = packed_stream(e, UPPER, pp_lanes(lanes))) {
+            sweep_stream(e, UPPER, *st, b, out, reset, gate, ctr, e->err.get() + kErrSweep);
             return;
         }
         ensure_pack(e, UPPER);
@@ -1690,6 +1877,11 @@ void sweep_dispatch(int lanes, Ext* e, const T* val, const double* b, double* ou
         sweep_blk_dispatch<T, UPPER>(lanes, e, val, b, out, reset, gate, ctr);
         return;
     }
+    if (mode == 0)
+        if (const SweepStream* st = auto_stream(e, UPPER)) {
+            sweep_stream(e, UPPER, *st, b, out, reset, gate, ctr, e->err.get() + kErrSweep);
+            return;
+        }
     switch (lanes) {
         case 1: sweep_one<1, T, UPPER>(e, val, b, out, reset, gate, ctr); break;
         case 2: sweep_one<2, T, UPPER>(e, val, b, out, reset, gate, ctr); break;
@@ -1768,8 +1960,12 @@ bool run_factor(Ext* e) {
     ++e->factor_version;
     gather_pack(e, e->pack_l, false);
     gather_pack(e, e->pack_u, true);
-    gather_stream(e, false);
-    gather_stream(e, true);
+    for (const bool upper : {false, true}) {
+        SweepStream& st = upper ? e->stream_u : e->stream_l;
+        SweepStream& at = upper ? e->auto_u : e->auto_l;
+        if (st.version == e->part_version && st.lds > 0) gather_stream(e, upper, st);
+        if (e->sweep_default && at.version == e->pattern_version && at.lds > 0) gather_stream(e, upper, at);
+    }
     if (ws_current(e, e->ws_l, e->ws_l.g)) gather_ws(e, e->ws_l);
     if (ws_current(e, e->ws_u, e->ws_u.g)) gather_ws(e, e->ws_u);
     return (err & 1) == 0 && e->factor_status == 0;
@@ -1795,7 +1991,8 @@ void show_algorithm(const lljbash::IluSolver* solver) {
 bool flags_in_output(Ext* e, bool upper) {
     const int mode = upper ? e->mode_u : e->mode_l;
     if (mode < 0 || mode > 3) return false;
-    return mode < 2 || e->nblk <= 0 || !ensure_stream(e, upper, pp_lanes(effective_lanes(e, upper)));
+    if (mode == 0) return !auto_stream(e, upper);
+    return mode == 1 || !packed_stream(e, upper, pp_lanes(effective_lanes(e, upper)));
 }
 
 // The forward sweep b -> y, then the backward sweep y -> x.  Each sweep
@@ -1831,6 +2028,7 @@ void arm_y(Ext* e) {
 void ilu_apply(Ext* e, const double* d_b, double* d_x, const int* gate) {
     need_setup(e);
     if (!e->factored) throw std::runtime_error("IluSolver: Factorize has not been called");
+    count_default_apply(e);
     arm_y(e);
     sweep_pair(e, d_b, d_x, e->y.get(), gate, e->ctr.get() + 4, nullptr);
     e->y_armed = flags_in_output(e, false);
@@ -2151,6 +2349,7 @@ int IluSolver::AutotuneSweeps(int reps, double* table, int cap) {
     Ext* e = pilu::need_setup(ext_);
     if (!e->factored) throw std::runtime_error("IluSolver: Factorize before AutotuneSweeps");
     reps = std::max(reps, 1);
+    e->sweep_default = false;
     hipStream_t s = e->stream;
     static const int kLanes[7] = {1, 2, 4, 8, 16, 32, 64};
     static const int kBlkLanes[4] = {4, 8, 16, 32};
@@ -2284,6 +2483,7 @@ void IluSolver::SetSweepMode(int mode_l, int mode_u, int blk_rows) {
     if (mode_l < 0 || mode_l > 5 || mode_u < 0 || mode_u > 5)
         throw std::runtime_error("sweep mode is 0, 1, 2, 3, 4 or 5");
     auto blocked = [](int m) { return (m >= 1 && m <= 3) || m == 5; };
+    e->sweep_default = false;
     if (blocked(mode_l) || blocked(mode_u)) pilu::use_blocks(e, blk_rows);
     e->mode_l = mode_l;
     e->mode_u = mode_u;
@@ -2305,6 +2505,7 @@ void IluSolver::SetSweepTiles(int mode_l, int mode_u, int tx, int ty, int tz) {
     Ext* e = pilu::need_setup(ext_);
     auto ok = [](int m) { return m == 0 || m == 2 || m == 3 || m == 5; };
     if (!ok(mode_l) || !ok(mode_u)) throw std::runtime_error("tiled sweeps use mode 0, 2, 3 or 5");
+    e->sweep_default = false;
     pilu::use_tiles(e, tx, ty, tz);
     e->mode_l = mode_l;
     e->mode_u = mode_u;

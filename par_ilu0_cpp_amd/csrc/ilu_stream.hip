@@ -554,7 +554,7 @@ void launch_st(Ext* e, const SweepStream& st, const T* sval, const double* b, do
     auto kern = k_sweep_st<G, T, UPPER>;
     PILU_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                  static_cast<int>(st.lds)));
-    kern<<<e->nblk, kStThreads, st.lds, e->stream>>>(
+    kern<<<st.nblk, kStThreads, st.lds, e->stream>>>(
         e->n, st.kptr.get(), st.cptr.get(), reinterpret_cast<const int2*>(st.irange.get()), st.mail.get(),
         static_cast<unsigned>(st.mail_words), st.gen.get(), static_cast<unsigned>(st.nchunk),
         reinterpret_cast<const uint2*>(st.scol.get()), sval, reinterpret_cast<const double2*>(st.sdiag.get()), b, out,
@@ -574,116 +574,105 @@ void sweep_st_t(Ext* e, const SweepStream& st, const T* sval, const double* b, d
 
 }  // namespace
 
-bool stream_applies(const Ext* e, bool upper, int G) {
-    const SweepStream& st = upper ? e->stream_u : e->stream_l;
-    if (e->nblk <= 0 || G < 2 || G > 16 || (upper ? e->max_up : e->max_lo) > G) return false;
-    return !(st.version == e->part_version && st.g == G && st.lds == 0);
+bool stream_width_fits(const Ext* e, bool upper, int G) {
+    return G >= 2 && G <= 16 && (upper ? e->max_up : e->max_lo) <= G;
 }
 
-bool ensure_stream(Ext* e, bool upper, int G) {
-    SweepStream& st = upper ? e->stream_u : e->stream_l;
-    if (!stream_applies(e, upper, G)) return false;
-    if (st.version != e->part_version || st.g != G) {
-        refuse_if_no_alloc(e, "sweep stream");
-        const int n = e->n, nblk = e->nblk, R = 64 / G, up = upper ? 1 : 0;
-        hipStream_t s = e->stream;
-        const int* perm = (upper ? e->bperm_u : e->bperm_l).get();
-        const int* blev = (upper ? e->blev_u : e->blev_l).get();
-        const int* loff = (upper ? e->loff_u : e->loff_l).get();
-        st.g = G;
-        st.version = e->part_version;
-        st.factors = -1;
-        st.lds = 0;
-        DevBuf<int> irefs(2 * static_cast<size_t>(nblk));
-        DevBuf<int> kinv(n), cnt(static_cast<size_t>(n) + 1), escan(static_cast<size_t>(n) + 1);
-        DevBuf<int> nch(static_cast<size_t>(nblk) + 1);
-        const size_t nb1 = static_cast<size_t>(nblk) + 1;
-        st.kptr.reserve(nb1);
-        st.cptr.reserve(nb1);
-        st.irange.reserve(2 * nb1);
-        k_st_kptr<<<grid_for(nblk + 1, 256), 256, 0, s>>>(nblk, blev, loff, st.kptr.get());
-        k_st_count<<<grid_for(static_cast<long>(n) + 1, 256), 256, 0, s>>>(n, up, perm, e->rp.get(), e->dg.get(),
-                                                                          e->ci.get(), e->block_of.get(), kinv.get(),
-                                                                          cnt.get());
-        PILU_HIP(hipGetLastError());
-        auto scan = [&](const int* in, int* out, size_t m) {
-            size_t bytes = 0;
-            PILU_HIP(rocprim::exclusive_scan(nullptr, bytes, in, out, 0, m, rocprim::plus<int>(), s));
-            e->sort_tmp.reserve(bytes);
-            PILU_HIP(rocprim::exclusive_scan(e->sort_tmp.get(), bytes, in, out, 0, m, rocprim::plus<int>(), s));
-        };
-        scan(cnt.get(), escan.get(), static_cast<size_t>(n) + 1);
-        k_st_chunks<<<nblk + 1, 256, 0, s>>>(nblk, R, blev, loff, nch.get());
-        PILU_HIP(hipGetLastError());
-        scan(nch.get(), st.cptr.get(), nb1);
-        // references per partition are bounded by the entries of one triangle
-        const int nref = read_word(escan.get() + n, s);
-        DevBuf<int> refs(std::max(nref, 1)), imp(std::max(nref, 1));
-        k_st_refs<<<grid_for(n, 256), 256, 0, s>>>(n, up, perm, e->rp.get(), e->dg.get(), e->ci.get(),
-                                                  e->block_of.get(), escan.get(), refs.get());
-        PILU_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_st_dedupe),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kStTableLds)));
-        k_st_dedupe<<<nblk, 1024, kStTableLds, s>>>(nblk, st.kptr.get(), escan.get(), refs.get(), imp.get(),
-                                                   reinterpret_cast<int2*>(irefs.get()));
-        PILU_HIP(hipGetLastError());
-        std::vector<int> h(4 * nb1);
-        PILU_HIP(hipMemcpyAsync(h.data(), st.kptr.get(), sizeof(int) * nb1, hipMemcpyDeviceToHost, s));
-        PILU_HIP(hipMemcpyAsync(h.data() + nb1, st.cptr.get(), sizeof(int) * nb1, hipMemcpyDeviceToHost, s));
-        PILU_HIP(hipMemcpyAsync(h.data() + 2 * nb1, irefs.get(), 2 * sizeof(int) * nblk, hipMemcpyDeviceToHost, s));
-        PILU_HIP(hipStreamSynchronize(s));
-        size_t lds = kStMinLds;
-        st.max_chunks = 0;
-        st.mail_words = 0;
-        for (int p = 0; p < nblk; ++p) {
-            const size_t rows = h[p + 1] - h[p], imps = h[2 * nb1 + 2 * p + 1];
-            h[2 * nb1 + 2 * p] = static_cast<int>(st.mail_words);
-            st.mail_words += static_cast<long>(imps);
-            lds = std::max(lds, 8 * (rows + imps + 2));
-            st.max_chunks = std::max(st.max_chunks, h[nb1 + p + 1] - h[nb1 + p]);
-        }
-        st.nchunk = h[nb1 + nblk];
-        PILU_HIP(hipMemcpyAsync(st.irange.get(), h.data() + 2 * nb1, 2 * sizeof(int) * nblk, hipMemcpyHostToDevice, s));
-        // every buffer has 32-bit byte offsets and the block fits the LDS (so
-        // its slots 15 bits); the packed factors take the partition otherwise
-        if (lds > kStMaxLds || st.nchunk > (1L << 31) / 512 || st.mail_words >= (1L << 28) || n >= (1 << 28)) return false;
-        const long nlanes = st.nchunk * 64;
-        int* rowlane = cnt.get();  // the counts have been scanned
-        DevBuf<int> chunks(2 * static_cast<size_t>(std::max<long>(st.nchunk, 1)));
-        st.scol.reserve(2 * std::max<long>(nlanes, 1));
-        st.ssrc.reserve(std::max<long>(nlanes, 1));
-        st.srow.reserve(static_cast<size_t>(std::max<long>(st.nchunk * R, 1)));
-        k_st_cut<<<nblk, 256, 0, s>>>(R, blev, loff, st.cptr.get(), reinterpret_cast<int2*>(chunks.get()));
-        auto fill = upper ? k_st_fill<true> : k_st_fill<false>;
-        if (nlanes > 0)
-            fill<<<grid_for(nlanes, 256), 256, 0, s>>>(
-                nlanes, G, nblk, reinterpret_cast<const int2*>(chunks.get()), st.cptr.get(), st.kptr.get(),
-                reinterpret_cast<const int2*>(irefs.get()), escan.get(), refs.get(), perm, kinv.get(), e->rp.get(),
-                e->dg.get(), e->ci.get(), e->block_of.get(),
-                reinterpret_cast<uint2*>(st.scol.get()), st.ssrc.get(), st.srow.get(),
-                rowlane);
-        // every import becomes a mailbox word its row's lanes store to
-        DevBuf<int> exported(static_cast<size_t>(n) + 1);
-        PILU_HIP(hipMemsetAsync(exported.get(), 0, sizeof(int) * (static_cast<size_t>(n) + 1), s));
-        if (st.mail_words > 0)
-            k_st_exports<<<nblk, 256, 0, s>>>(G, reinterpret_cast<const int2*>(irefs.get()),
-                                              reinterpret_cast<const int2*>(st.irange.get()), imp.get(), rowlane,
-                                              exported.get(), reinterpret_cast<uint2*>(st.scol.get()),
-                                              exported.get() + n);
-        st.mail.reserve(2 * static_cast<size_t>(std::max(st.mail_words, 1L)));
-        st.gen.reserve(1);
-        PILU_HIP(hipMemsetAsync(st.gen.get(), 0, sizeof(int), s));
-        k_st_arm<<<grid_for(2 * st.mail_words, 256 * 8), 256, 0, s>>>(2 * st.mail_words, st.mail.get(), nullptr);
-        PILU_HIP(hipGetLastError());
-        if (read_word(exported.get() + n, s) != 0) return false;  // a row with more importing blocks than lanes
-        st.lds = lds;
+bool build_stream(Ext* e, bool upper, int G, const StreamSchedule& sc, SweepStream& st) {
+    refuse_if_no_alloc(e, "sweep stream");
+    const int n = e->n, nblk = sc.nblk, R = 64 / G, up = upper ? 1 : 0;
+    hipStream_t s = e->stream;
+    const int *perm = sc.perm, *blev = sc.blev, *loff = sc.loff, *block_of = sc.block_of;
+    st.g = G;
+    st.nblk = nblk;
+    st.factors = -1;
+    st.lds = 0;
+    DevBuf<int> irefs(2 * static_cast<size_t>(nblk));
+    DevBuf<int> kinv(n), cnt(static_cast<size_t>(n) + 1), escan(static_cast<size_t>(n) + 1);
+    DevBuf<int> nch(static_cast<size_t>(nblk) + 1);
+    const size_t nb1 = static_cast<size_t>(nblk) + 1;
+    st.kptr.reserve(nb1);
+    st.cptr.reserve(nb1);
+    st.irange.reserve(2 * nb1);
+    k_st_kptr<<<grid_for(nblk + 1, 256), 256, 0, s>>>(nblk, blev, loff, st.kptr.get());
+    k_st_count<<<grid_for(static_cast<long>(n) + 1, 256), 256, 0, s>>>(n, up, perm, e->rp.get(), e->dg.get(),
+                                                                      e->ci.get(), block_of, kinv.get(),
+                                                                      cnt.get());
+    PILU_HIP(hipGetLastError());
+    auto scan = [&](const int* in, int* out, size_t m) {
+        size_t bytes = 0;
+        PILU_HIP(rocprim::exclusive_scan(nullptr, bytes, in, out, 0, m, rocprim::plus<int>(), s));
+        e->sort_tmp.reserve(bytes);
+        PILU_HIP(rocprim::exclusive_scan(e->sort_tmp.get(), bytes, in, out, 0, m, rocprim::plus<int>(), s));
+    };
+    scan(cnt.get(), escan.get(), static_cast<size_t>(n) + 1);
+    k_st_chunks<<<nblk + 1, 256, 0, s>>>(nblk, R, blev, loff, nch.get());
+    PILU_HIP(hipGetLastError());
+    scan(nch.get(), st.cptr.get(), nb1);
+    // references per partition are bounded by the entries of one triangle
+    const int nref = read_word(escan.get() + n, s);
+    DevBuf<int> refs(std::max(nref, 1)), imp(std::max(nref, 1));
+    k_st_refs<<<grid_for(n, 256), 256, 0, s>>>(n, up, perm, e->rp.get(), e->dg.get(), e->ci.get(),
+                                              block_of, escan.get(), refs.get());
+    PILU_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_st_dedupe),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kStTableLds)));
+    k_st_dedupe<<<nblk, 1024, kStTableLds, s>>>(nblk, st.kptr.get(), escan.get(), refs.get(), imp.get(),
+                                               reinterpret_cast<int2*>(irefs.get()));
+    PILU_HIP(hipGetLastError());
+    std::vector<int> h(4 * nb1);
+    PILU_HIP(hipMemcpyAsync(h.data(), st.kptr.get(), sizeof(int) * nb1, hipMemcpyDeviceToHost, s));
+    PILU_HIP(hipMemcpyAsync(h.data() + nb1, st.cptr.get(), sizeof(int) * nb1, hipMemcpyDeviceToHost, s));
+    PILU_HIP(hipMemcpyAsync(h.data() + 2 * nb1, irefs.get(), 2 * sizeof(int) * nblk, hipMemcpyDeviceToHost, s));
+    PILU_HIP(hipStreamSynchronize(s));
+    size_t lds = kStMinLds;
+    st.max_chunks = 0;
+    st.mail_words = 0;
+    for (int p = 0; p < nblk; ++p) {
+        const size_t rows = h[p + 1] - h[p], imps = h[2 * nb1 + 2 * p + 1];
+        h[2 * nb1 + 2 * p] = static_cast<int>(st.mail_words);
+        st.mail_words += static_cast<long>(imps);
+        lds = std::max(lds, 8 * (rows + imps + 2));
+        st.max_chunks = std::max(st.max_chunks, h[nb1 + p + 1] - h[nb1 + p]);
     }
-    if (e->factored && st.factors != e->factor_version) gather_stream(e, upper);
+    st.nchunk = h[nb1 + nblk];
+    // every buffer has 32-bit byte offsets and the block fits the LDS (so
+    // its slots 15 bits); the packed factors take the partition otherwise
+    if (lds > kStMaxLds || st.nchunk > (1L << 31) / 512 || st.mail_words >= (1L << 28) || n >= (1 << 28))
+        return false;
+    PILU_HIP(hipMemcpyAsync(st.irange.get(), h.data() + 2 * nb1, 2 * sizeof(int) * nblk, hipMemcpyHostToDevice, s));
+    const long nlanes = st.nchunk * 64;
+    int* rowlane = cnt.get();  // the counts have been scanned
+    DevBuf<int> chunks(2 * static_cast<size_t>(std::max<long>(st.nchunk, 1)));
+    st.scol.reserve(2 * std::max<long>(nlanes, 1));
+    st.ssrc.reserve(std::max<long>(nlanes, 1));
+    st.srow.reserve(static_cast<size_t>(std::max<long>(st.nchunk * R, 1)));
+    k_st_cut<<<nblk, 256, 0, s>>>(R, blev, loff, st.cptr.get(), reinterpret_cast<int2*>(chunks.get()));
+    auto fill = upper ? k_st_fill<true> : k_st_fill<false>;
+    if (nlanes > 0)
+        fill<<<grid_for(nlanes, 256), 256, 0, s>>>(
+            nlanes, G, nblk, reinterpret_cast<const int2*>(chunks.get()), st.cptr.get(), st.kptr.get(),
+            reinterpret_cast<const int2*>(irefs.get()), escan.get(), refs.get(), perm, kinv.get(), e->rp.get(),
+            e->dg.get(), e->ci.get(), block_of, reinterpret_cast<uint2*>(st.scol.get()), st.ssrc.get(),
+            st.srow.get(), rowlane);
+    // every import becomes a mailbox word its row's lanes store to
+    DevBuf<int> exported(static_cast<size_t>(n) + 1);
+    PILU_HIP(hipMemsetAsync(exported.get(), 0, sizeof(int) * (static_cast<size_t>(n) + 1), s));
+    if (st.mail_words > 0)
+        k_st_exports<<<nblk, 256, 0, s>>>(G, reinterpret_cast<const int2*>(irefs.get()),
+                                          reinterpret_cast<const int2*>(st.irange.get()), imp.get(), rowlane,
+                                          exported.get(), reinterpret_cast<uint2*>(st.scol.get()),
+                                          exported.get() + n);
+    st.mail.reserve(2 * static_cast<size_t>(std::max(st.mail_words, 1L)));
+    st.gen.reserve(1);
+    PILU_HIP(hipMemsetAsync(st.gen.get(), 0, sizeof(int), s));
+    k_st_arm<<<grid_for(2 * st.mail_words, 256 * 8), 256, 0, s>>>(2 * st.mail_words, st.mail.get(), nullptr);
+    PILU_HIP(hipGetLastError());
+    if (read_word(exported.get() + n, s) != 0) return false;  // a row with more importing blocks than lanes
+    st.lds = lds;
     return true;
 }
 
-void gather_stream(Ext* e, bool upper) {
-    SweepStream& st = upper ? e->stream_u : e->stream_l;
-    if (st.version != e->part_version || st.lds == 0) return;
+void gather_stream(Ext* e, bool upper, SweepStream& st) {
     refuse_if_no_alloc(e, "sweep stream values");
     const long nlanes = st.nchunk * 64, nrow = st.nchunk * (64 / st.g);
     if (upper) st.sdiag.reserve(2 * static_cast<size_t>(std::max<long>(nrow, 1)));
@@ -702,10 +691,9 @@ void gather_stream(Ext* e, bool upper) {
     st.factors = e->factor_version;
 }
 
-void sweep_stream(Ext* e, bool upper, const double* b, double* out, double* reset, const int* gate, int* ctr,
-                  int* err) {
-    const SweepStream& st = upper ? e->stream_u : e->stream_l;
-    if (st.version != e->part_version || st.lds == 0 || st.factors != e->factor_version)
+void sweep_stream(Ext* e, bool upper, const SweepStream& st, const double* b, double* out, double* reset,
+                  const int* gate, int* ctr, int* err) {
+    if (st.lds == 0 || st.factors != e->factor_version)
         throw std::runtime_error("stream sweep: stream missing (factorize before sweeping)");
     if (e->precision == 32) {
         if (upper) sweep_st_t<float, true>(e, st, st.sval32.get(), b, out, gate, ctr, err);

@@ -5,22 +5,29 @@
 
 namespace pilu {
 
-// Whether the current partition may be swept over a stream with G lanes per
-// row: one lane per entry, and no earlier attempt found the block too large
-// for the LDS.
-bool stream_applies(const lljbash::IluSolver::Ext* e, bool upper, int G);
+// Rows in sweep order and how they are grouped (device arrays): rows of block
+// p (processing order) and one local level are perm[loff[g] .. loff[g + 1]),
+// g in [blev[p], blev[p + 1]); blev has nblk + 1 entries.
+struct StreamSchedule {
+    const int *perm, *blev, *loff, *block_of;
+    int nblk;
+};
 
-// Builds the stream (and its values, once factored) where it is missing or
-// stale; false where the partition has to be swept otherwise.
-bool ensure_stream(lljbash::IluSolver::Ext* e, bool upper, int G);
+// Whether every row of the direction has at most one entry per lane.
+bool stream_width_fits(const lljbash::IluSolver::Ext* e, bool upper, int G);
 
-// Refreshes the values of a current stream from the factors.
-void gather_stream(lljbash::IluSolver::Ext* e, bool upper);
+// Builds the pattern part of a stream for G lanes per row
+// (stream_width_fits); false, with st.lds == 0, where a block does not fit
+// the LDS or a row is imported by more blocks than it has lanes for.
+bool build_stream(lljbash::IluSolver::Ext* e, bool upper, int G, const StreamSchedule& sc, SweepStream& st);
 
-// One sweep (ensure_stream has returned true for this direction).  reset, if
-// given, is filled with kPending after it.
-void sweep_stream(lljbash::IluSolver::Ext* e, bool upper, const double* b, double* out, double* reset, const int* gate,
-                  int* ctr, int* err);
+// Refreshes the values of a built stream from the factors.
+void gather_stream(lljbash::IluSolver::Ext* e, bool upper, SweepStream& st);
+
+// One sweep over a stream whose values are current.  reset, if given, is
+// filled with kPending after it.
+void sweep_stream(lljbash::IluSolver::Ext* e, bool upper, const SweepStream& st, const double* b, double* out,
+                  double* reset, const int* gate, int* ctr, int* err);
 
 // Raised when a sweep structure is missing during a no-allocation apply.
 void refuse_if_no_alloc(const lljbash::IluSolver::Ext* e, const char* what);

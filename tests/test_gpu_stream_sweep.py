@@ -109,3 +109,65 @@ def test_row_imported_by_many_blocks(blocks, stream):
     for _ in range(2):
         assert np.array_equal(ilu.Substitute(b), want)
     assert ("lds_bytes" in ilu.Schedule()["pack_l"]) is stream
+
+
+def grid_matrix(nx, ny, nz, lof, oracle):
+    """7-point (5-point for one plane) operator with its ILU(lof) pattern."""
+    rng = np.random.default_rng(nx + 10 * ny + 100 * nz)
+    rp, ci, va = [0], [], []
+    for i in range(nx * ny * nz):
+        x, y, z = i % nx, (i // nx) % ny, i // (nx * ny)
+        row = [i]
+        for p, m, s in ((x, nx, 1), (y, ny, nx), (z, nz, nx * ny)):
+            row += [i - s] * (p > 0) + [i + s] * (p + 1 < m)
+        ci += sorted(row)
+        va += [7.0 if c == i else float(rng.uniform(-1, -0.1)) for c in sorted(row)]
+        rp.append(len(ci))
+    o = oracle.iluk_symbolic(np.array(rp, np.int32), np.array(ci, np.int32), np.array(va), lof)
+    return o[0], o[1], o[3]
+
+
+@pytest.mark.parametrize("shape,lof", [((40, 30, 1), 0), ((150, 131, 1), 1), ((21, 20, 19), 0), ((17, 13, 30), 1),
+                                       ((2, 90, 100), 1), ((7, 1, 1), 0)])
+@pytest.mark.parametrize("bits", [64, 32])
+def test_default_sweeps_keep_their_bits(oracle, shape, lof, bits):
+    """A solver whose sweep shape is never set changes to chunk streams after
+    a few applies (one workgroup, or tiles of the grid its pattern is taken
+    for) and returns to level rows when a shape is set; the reported
+    configuration and every result stay the same, also after a new
+    factorization."""
+    rp, ci, va = grid_matrix(*shape, lof, oracle)
+    n = rp.size - 1
+    ilu = factored(rp, ci, va, bits)
+    before = ilu.SweepConfig()
+    b = np.random.default_rng(5).uniform(-1, 1, n)
+    first = ilu.Substitute(b)
+    for _ in range(5):
+        assert np.array_equal(ilu.Substitute(b), first)
+    assert ilu.SweepConfig() == before
+    fac, dg, _ = oracle.ilu_factorize(rp, ci, va)
+    if bits == 32:
+        fac = fac.astype(np.float32).astype(np.float64)
+    assert np.array_equal(first, oracle.substitute_lanes(rp, ci, dg, fac, b, before["lanes_l"]))
+    P.fill_csr(ilu.GetMatrix(), rp, ci, va * 1.25)
+    assert ilu.Factorize() == 0
+    again = ilu.Substitute(b)
+    y = ilu.Trsv(False, 1.0, b)
+    z = ilu.Trsv(True, 1.0, y)
+    assert np.array_equal(z, again)
+    ilu.SetSweepMode(0, 0, 0)
+    assert np.array_equal(ilu.Substitute(b), again)
+    ilu.SetSweepLanes(1, 1)
+    assert np.allclose(ilu.Substitute(b), again, rtol=1e-10, atol=1e-13 if bits == 64 else 1e-10)
+
+
+def test_default_sweeps_without_a_grid():
+    """Short rows at irregular offsets: one workgroup where the matrix fits
+    one, level rows where it does not."""
+    for n in (9000, 20000):
+        rp, ci, va = banded(n, 3, 400, seed=n)
+        ilu = factored(rp, ci, va)
+        b = np.random.default_rng(6).uniform(-1, 1, n)
+        first = ilu.Substitute(b)
+        for _ in range(4):
+            assert np.array_equal(ilu.Substitute(b), first)
