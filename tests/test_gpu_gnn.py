@@ -147,3 +147,38 @@ def test_trained_network_beats_plain_ilu(seed):
     assert res <= 1.01e-8 and res0 <= 1.01e-8
     assert its <= 0.55 * its0, (its, its0)
     assert its <= itsc + 2, (its, itsc)
+
+
+@pytest.mark.parametrize("n", [1, 15, 64, 65, 700])
+def test_uneven_rows_match_oracle(n):
+    """Rows with no edges and rows of 1 to 40 of them (more than one round of
+    gathered edges, feature blocks past their LDS stage), and row counts around
+    the 16-row and 64-row tiles: prediction and gradients against the oracle."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    rows = [set() for _ in range(n)]
+    for i in range(n):
+        for j in rng.integers(0, n, size=int(rng.integers(0, 21))):
+            rows[i].add(int(j))
+            rows[int(j)].add(i)
+    for i in range(n):
+        rows[i].add(i)
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    ci = np.concatenate([sorted(r) for r in rows]).astype(np.int32)
+    va = rng.uniform(-1.0, -0.1, ci.size)
+    va[ci == np.repeat(np.arange(n), np.diff(rp))] = rng.uniform(10.0, 20.0, n)
+    p = rng.normal(0, 0.25, G.N_PARAMS).astype(np.float32)
+    t = rng.uniform(0.3, 0.95, n).astype(np.float32)
+    net = Gnn(p)
+    rpt, cit, tmap = transpose_map(rp, ci)
+    d = dev(rp, ci, va, rpt, cit, tmap, t)
+    om = torch.zeros(n, dtype=torch.float32, device="cuda")
+    net.predict(n, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), om.data_ptr())
+    feat, w = G.features(rp, ci, va)
+    ref, _, _ = G.forward(p.astype(np.float64), rp, ci, feat, w, use_bf16=True)
+    assert np.max(np.abs(om.cpu().numpy() - ref)) <= 5e-3
+    loss, g = net.gradients(n, *[x.data_ptr() for x in d])
+    lref, gref = G.loss_grad(p.astype(np.float64), rp, ci, feat, w, t.astype(np.float64), True)
+    assert loss == pytest.approx(lref, rel=2e-2)
+    assert np.linalg.norm(g - gref) <= 3e-2 * np.linalg.norm(gref)
