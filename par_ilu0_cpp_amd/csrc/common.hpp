@@ -198,6 +198,25 @@ __device__ __forceinline__ bool group_all(bool pred) {
     }
 }
 
+// s / d with rc = 1 / d rounded to nearest: q = s rc, then one correction
+// q + (s - q d) rc, correctly rounded (Markstein 1990, IBM J. Res. Dev. 34)
+// as long as no intermediate leaves the normal range.  rc is 0 where d is
+// outside 2^+-200 (recip_for); s outside 2^+-766 (zero, infinity and NaN
+// included) in one of `lanes` takes the wave through the division itself.
+__device__ __forceinline__ double recip_for(double d) {
+    const unsigned e = (static_cast<unsigned>(__double2hiint(d)) >> 20) & 0x7ffu;
+    return e - (1023u - 200u) <= 400u ? 1.0 / d : 0.0;
+}
+
+__device__ __forceinline__ double divide_by(double s, double d, double rc, uint64_t lanes) {
+    const unsigned e = (static_cast<unsigned>(__double2hiint(s)) >> 20) & 0x7ffu;
+    const uint64_t slow = (__ballot(e - 257u > 1532u) | __ballot(rc == 0.0)) & lanes;
+    const double q = s * rc;
+    double r = fma(fma(-q, d, s), rc, q);
+    if (__builtin_expect(slow != 0, 0)) r = s / d;
+    return r;
+}
+
 __device__ __forceinline__ void spin_pause() { __builtin_amdgcn_s_sleep(1); }
 
 // Watchdog for sync-free waits: a wait that outlives `limit` ticks of the
@@ -212,6 +231,38 @@ struct Watchdog {
     __device__ explicit Watchdog(uint64_t lim) : start(wall_clock64()), limit(lim) {}
     __device__ bool expired() const { return wall_clock64() - start > limit; }
 };
+
+// Back substitution of the (i + 1) x (i + 1) upper triangle hh (columns `ld`
+// apart) by one wave, rs in place (src/gmres.cpp:265-272): the wave copies the
+// triangle to `tri` (LDS, room for kBackMax columns) and its first lane solves
+// row by row from there, in the same order; larger triangles are read where
+// they are.  From memory a thread took 140 us for 50 columns.
+constexpr int kBackMax = 64;
+__device__ __forceinline__ void back_substitute(int i, const double* hh, long ld, double* rs, double* tri) {
+    const int lane = threadIdx.x & 63;
+    const bool staged = i < kBackMax;
+    if (staged)
+        for (int j = 0; j <= i; ++j)
+            for (int k = lane; k <= j; k += 64) tri[j * kBackMax + k] = hh[j * ld + k];
+    double* const x = tri + kBackMax * kBackMax;
+    for (int k = lane; staged && k <= i; k += 64) x[k] = rs[k];
+    __syncthreads();
+    auto solve = [i](const double* t, long st, double* r) {
+        r[i] = r[i] / t[i * st + i];
+        for (int ii = i - 1; ii >= 0; --ii) {
+            double v = r[ii];
+            for (int j = ii + 1; j <= i; ++j) v -= t[j * st + ii] * r[j];
+            r[ii] = v / t[ii * st + ii];
+        }
+    };
+    if (lane == 0) {
+        if (staged) solve(tri, kBackMax, x);  // apart, so that these are LDS reads
+        else solve(hh, ld, rs);
+    }
+    __syncthreads();
+    for (int k = lane; staged && k <= i; k += 64) rs[k] = x[k];
+}
+constexpr int kBackLds = kBackMax * (kBackMax + 1);  // doubles
 
 // Ticks of the device wall clock in `seconds` (host side).
 uint64_t watchdog_ticks(double seconds);

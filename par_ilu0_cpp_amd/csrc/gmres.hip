@@ -326,17 +326,11 @@ __global__ void k_arnoldi_finish(GmresCtl* ctl, const double* part, const double
 }
 
 // Upper-triangular solve for the step coefficients (src/gmres.cpp:265-272).
-__global__ void k_backsolve(GmresCtl* ctl, double* hh) {
+__global__ __launch_bounds__(64) void k_backsolve(GmresCtl* ctl, double* hh) {
+    __shared__ double s_tri[kBackLds];
     if (ctl->status == 2 || ctl->i < 0) return;
     const int im = ctl->im, im1 = im + 1;
-    const int i = ctl->i;
-    double* rs = hh + static_cast<long>(im1) * im + 2 * im1;
-    rs[i] = rs[i] / hh[static_cast<long>(i) * im1 + i];
-    for (int ii = i - 1; ii >= 0; --ii) {
-        double t = rs[ii];
-        for (int j = ii + 1; j <= i; ++j) t -= hh[static_cast<long>(j) * im1 + ii] * rs[j];
-        rs[ii] = t / hh[static_cast<long>(ii) * im1 + ii];
-    }
+    back_substitute(ctl->i, hh, im1, hh + static_cast<long>(im1) * im + 2 * im1, s_tri);
 }
 
 // sol += sum_j rs_j z_j, j = 0..i, applied in ascending j per entry
@@ -672,7 +666,7 @@ std::pair<bool, int> solve_core(GExt* e, IluSolver* ilu, const std::function<voi
                 if (!e->snap[(i - 1) & 1].cycle_active) break;
             }
         }
-        pilu::k_backsolve<<<1, 1, 0, s>>>(dctl, hh);
+        pilu::k_backsolve<<<1, 64, 0, s>>>(dctl, hh);
         pilu::k_update<<<pilu::kVecBlocks, pilu::kVecThreads, 0, s>>>(n, z, dctl, hh, sol);
         PILU_HIP(hipGetLastError());
         PILU_HIP(hipMemcpyAsync(&h, dctl, sizeof(h), hipMemcpyDeviceToHost, s));

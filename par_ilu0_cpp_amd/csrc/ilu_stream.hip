@@ -108,25 +108,6 @@ __device__ __forceinline__ uint64_t wait_lds(unsigned at, const Watchdog& wd, bo
     return bits;
 }
 
-// s / d with rc = 1 / d rounded to nearest: q = s rc, then one correction
-// q + (s - q d) rc, correctly rounded (Markstein 1990, IBM J. Res. Dev. 34)
-// as long as no intermediate leaves the normal range.  rc is 0 where d is
-// outside 2^+-200 (st_recip); s outside 2^+-766 (zero, infinity and NaN
-// included) in one of `lanes` takes the wave through the division itself.
-__device__ __forceinline__ double st_recip(double d) {
-    const unsigned e = (static_cast<unsigned>(__double2hiint(d)) >> 20) & 0x7ffu;
-    return e - (1023u - 200u) <= 400u ? 1.0 / d : 0.0;
-}
-
-__device__ __forceinline__ double st_divide(double s, double d, double rc, uint64_t lanes) {
-    const unsigned e = (static_cast<unsigned>(__double2hiint(s)) >> 20) & 0x7ffu;
-    const uint64_t slow = (__ballot(e - 257u > 1532u) | __ballot(rc == 0.0)) & lanes;
-    const double q = s * rc;
-    double r = fma(fma(-q, d, s), rc, q);
-    if (__builtin_expect(slow != 0, 0)) r = s / d;
-    return r;
-}
-
 // One lane of a chunk: where its x and its row's x sit in LDS (slots in bits
 // 0..14 and 15..29), and a byte offset: lane 0 of a row: the row in b and
 // out; the other lanes: a mailbox word the row's result goes to.
@@ -282,7 +263,7 @@ __global__ __launch_bounds__(kStThreads) void k_sweep_st(int n, const int* __res
                 if (p + u < npass) {
                     const uint64_t bits = wait_lds(lds0 + (a.p.x & 0x7fffu) * 8u, wd, timed_out);
                     const double sum = group_sum<G>(fma(-__longlong_as_double(bits), static_cast<double>(r.v), r.b));
-                    const double x = UPPER ? st_divide(sum, r.d.x, r.d.y, first_lanes) : sum;
+                    const double x = UPPER ? divide_by(sum, r.d.x, r.d.y, first_lanes) : sum;
                     if (first) lds_put(xs, (a.p.x >> 15) * 8u, x);
                     asm volatile("" ::: "memory");  // the LDS word first: the next level waits for it
                     const double xg = group_first<G>(x);
@@ -544,7 +525,7 @@ __global__ void k_st_gather(long nlanes, const int* __restrict__ src, const T* _
         for (long k = i0; k < nrow; k += stride) {
             const int row = srow[k];
             const double d = row >= 0 ? static_cast<double>(fac[dg[row]]) : 1.0;
-            sdiag[k] = make_double2(d, st_recip(d));
+            sdiag[k] = make_double2(d, recip_for(d));
         }
 }
 

@@ -137,3 +137,61 @@ def test_batched_systems_are_independent_of_their_neighbours():
             ref_x, ref_its = (Xf, its_f[0]) if a is fast else (Xs, its_s[0])
             assert np.array_equal(its[k], ref_its)
             assert np.array_equal(X[sp[k]:sp[k + 1]], ref_x)
+
+
+def _general(n, per_row, band, seed):
+    """Nonsymmetric, diagonally dominant, up to per_row entries on either side."""
+    rng = np.random.default_rng(seed)
+    rows = []
+    for i in range(n):
+        lo = rng.integers(max(0, i - band), i + 1, size=int(rng.integers(0, per_row + 1)))
+        hi = rng.integers(i, min(n, i + band), size=int(rng.integers(0, per_row + 1))) if i + 1 < n else []
+        rows.append(sorted({int(j) for j in lo} | {int(j) for j in hi} | {i}))
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    ci = np.concatenate(rows).astype(np.int32)
+    va = rng.uniform(-1.0, 1.0, ci.size)
+    va[ci == np.repeat(np.arange(n), np.diff(rp))] = 1.5 * per_row + 1.0
+    return gen.Csr(n, rp, ci, va)
+
+
+@pytest.mark.parametrize("nrhs", [1, 4, 8])
+@pytest.mark.parametrize("case", ["narrow", "wide_rows", "far", "one_row", "long_rows"])
+def test_batched_sweep_forms_match_per_system_oracle(oracle, nrhs, case):
+    """What decides how a batch is swept and orthogonalised: rows of 2, 4 and
+    more entries per direction, dependencies that leave the LDS ring, systems
+    of one row and of several chunks, an odd restart length and restarts."""
+    if case == "narrow":
+        mats = [_general(n, 2, 30, n) for n in (257, 64, 1, 2100)]
+    elif case == "wide_rows":
+        mats = [_general(n, 4, 50, n) for n in (300, 513)]
+    elif case == "far":
+        mats = [_general(n, 2, n, n) for n in (9000, 40)]
+    elif case == "one_row":
+        mats = [gen.Csr(1, np.array([0, 1], np.int32), np.array([0], np.int32), np.array([2.0]))] * 9
+    else:
+        mats = [_general(n, 9, 40, n) for n in (200, 777)]
+    n = sum(m.n for m in mats)
+    rhs = np.random.default_rng(7).uniform(-1, 1, (n, nrhs))
+    rp, ci, va, sp = P.block_diagonal(mats)
+    d = [torch_dev(v) for v in (rp, ci, va, rhs)]
+    x = torch_dev(np.zeros((n, nrhs)))
+    bg = P.BatchGmres()
+    assert bg.Setup(n, d[0].data_ptr(), d[1].data_ptr(), 0, sp, nrhs) == ci.size
+    assert bg.Factorize(d[2].data_ptr()) == 0
+    _, its, conv, rel = bg.Solve(*[v.data_ptr() for v in d], x.data_ptr(), 1e-10, 5, 300)
+    X = x.cpu().numpy()
+    assert conv.all() and np.all(rel <= 1.01e-10)
+    for k, a in enumerate(mats):
+        fac, dg, _ = oracle.ilu_factorize(a.row_ptr, a.col_idx, a.value)
+        for r in range(nrhs):
+            b = np.ascontiguousarray(rhs[sp[k]:sp[k + 1], r])
+            ok, want, xo, _ = oracle.gmres((a.row_ptr, a.col_idx, a.value), b, 1e-10 * np.linalg.norm(b), 5, 300,
+                                           factors=(a.row_ptr, a.col_idx, dg, fac))
+            assert ok and abs(int(its[k, r]) - want) <= 1
+            assert np.linalg.norm(X[sp[k]:sp[k + 1], r] - xo) <= 1e-8 * np.linalg.norm(xo)
+
+
+def torch_dev(v):
+    import torch
+
+    return torch.from_numpy(np.ascontiguousarray(v)).cuda()
