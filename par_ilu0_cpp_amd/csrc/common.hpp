@@ -174,6 +174,23 @@ __device__ __forceinline__ double group_sum(double v) {
     return v;
 }
 
+// Sum over the wave, in every lane: within rows of 16 by DPP shifts, then the
+// rows' sums in order (a fixed order; no LDS traffic, where a shuffle
+// butterfly takes six dependent LDS round trips).
+__device__ __forceinline__ double wave_total(double v) {
+    v += dpp_row_shl<8>(v);
+    v += dpp_row_shl<4>(v);
+    v += dpp_row_shl<2>(v);
+    v += dpp_row_shl<1>(v);
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < 64; k += 16) {
+        const int lo = __builtin_amdgcn_readlane(__double2loint(v), k), hi = __builtin_amdgcn_readlane(__double2hiint(v), k);
+        t += __hiloint2double(hi, lo);
+    }
+    return t;
+}
+
 template <int G>
 __device__ __forceinline__ int group_max(int v) {
 #pragma unroll

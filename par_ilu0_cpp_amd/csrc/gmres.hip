@@ -7,7 +7,8 @@
 // breakdown and NaN checks) runs in single-block kernels on a small control
 // block in device memory, and every vector kernel of a step is gated by the
 // control block's step flag.  The host only looks at the control block one
-// step behind (to stop enqueuing) and at the end of each cycle.
+// step behind (to stop enqueuing; a word in its memory, written at a step's end) and
+// at the end of each cycle.
 #include <atomic>
 #include <chrono>
 #include <cmath>
@@ -37,7 +38,14 @@ struct GmresCtl {
     double tol;
     double beta;       // latest residual estimate
     double inv;        // scale for the vector just normalised
+    // device clock: start of the preconditioner apply and of the SpMV under
+    // way; ticks spent in either so far (GmresStat's timers)
+    uint64_t t_precon, t_mv, ticks_precon, ticks_mv;
 };
+
+// Word of the host's view of a step: kStepDone once the step has run, plus
+// whether the cycle goes on.
+constexpr int kStepDone = 2;
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -62,10 +70,10 @@ __device__ double block_sum(double v) {
     return s_total;
 }
 
-// Sum of kVecBlocks partials, identical in every block.
-__device__ double sum_partials(const double* part) {
+// Sum of np (<= kVecBlocks) partials, identical in every block.
+__device__ double sum_partials(const double* part, int np) {
     double v = 0.0;
-    for (int k = threadIdx.x; k < kVecBlocks; k += blockDim.x) v += part[k];
+    for (int k = threadIdx.x; k < np; k += blockDim.x) v += part[k];
     return block_sum(v);
 }
 
@@ -79,8 +87,13 @@ __global__ __launch_bounds__(kVecThreads) void k_spmv(int n, const int* __restri
                                                       const double* __restrict__ x, double beta,
                                                       const double* yin, double* y,
                                                       const double* __restrict__ dotv, bool nrm,
-                                                      double* part, const int* gate) {
+                                                      double* part, const int* gate, GmresCtl* clock) {
     if (gate && *gate == 0) return;
+    if (clock && blockIdx.x == 0 && threadIdx.x == 0) {
+        const uint64_t t = wall_clock64();
+        if (gate) clock->ticks_precon += t - clock->t_precon;
+        clock->t_mv = t;
+    }
     constexpr int R = 64 / G;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -110,10 +123,11 @@ __global__ __launch_bounds__(kVecThreads) void k_spmv(int n, const int* __restri
 //   w -= h v_j;  then partials of (vnext, w) or of (w, w) if vnext is null.
 __global__ __launch_bounds__(kVecThreads) void k_mgs(int n, const double* __restrict__ vj, double* w,
                                                      const double* __restrict__ vnext,
-                                                     const double* part_in, double* part_out,
-                                                     double* hout, const int* gate) {
+                                                     const double* part_in, int np, double* part_out,
+                                                     double* hout, const int* gate, GmresCtl* clock) {
     if (gate && *gate == 0) return;
-    const double h = sum_partials(part_in);
+    if (clock && blockIdx.x == 0 && threadIdx.x == 0) clock->ticks_mv += wall_clock64() - clock->t_mv;
+    const double h = sum_partials(part_in, np);
     if (blockIdx.x == 0 && threadIdx.x == 0) *hout = h;
     double acc = 0.0;
     const long stride = static_cast<long>(gridDim.x) * blockDim.x;
@@ -136,36 +150,147 @@ __global__ __launch_bounds__(kVecThreads) void k_mgs(int n, const double* __rest
 // stays in registers for the next term: each basis vector is read once.
 // h_0 comes from the SpMV's kVecBlocks partials as in the per-term path.
 // Finally w is scaled by 1 / ||w|| unless ||w|| <= 1e-16 (the breakdown
-// of src/gmres.cpp:228-233) and ||w|| is left in *tnorm.  The grid must be
-// co-resident (cooperative launch); partial slots come in two generations
-// (step parity), each step re-arming the other one.  Every wait carries the
-// watchdog.
+// of src/gmres.cpp:228-233), and workgroup 0 ends the step (rotations, next
+// gate, the host's word), which cost three launches and a copy before.  The
+// grid must be co-resident (cooperative launch); partial slots come in two
+// generations (step parity), each step re-arming the other one.  Every wait
+// carries the watchdog.
 // ---------------------------------------------------------------------
 constexpr int kMgsThreads = 512;
 
-__device__ double block_sum512(double v) {
-    __shared__ double s_part[kMgsThreads / 64];
-    __shared__ double s_total;
-    v = wave_sum(v);
+// Sum over a workgroup of W waves, in every thread: wave totals, then in wave
+// order.  `buf` (2 W doubles of LDS) alternates by `turn`, so one barrier per
+// sum is enough.
+template <int W>
+__device__ __forceinline__ double block_total(double v, double* buf, int& turn) {
+    double* b = buf + (turn & 1) * W;
+    ++turn;
+    v = wave_total(v);
+    if ((threadIdx.x & 63) == 0) b[threadIdx.x >> 6] = v;
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = v;
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < W; ++k) t += b[k];
+    return t;
+}
+
+// Loop condition of the Krylov loop (src/gmres.cpp:199) for step i.
+__device__ __forceinline__ void step_gate(GmresCtl* ctl, int i) {
+    if (ctl->cycle_active && ctl->beta > ctl->tol) {
+        const int before = ctl->its++;
+        if (before < ctl->maxits) {
+            ctl->step_active = 1;
+            ctl->i = i;
+            ctl->t_precon = wall_clock64();
+            return;
+        }
+    }
+    ctl->step_active = 0;
+    ctl->cycle_active = 0;
+}
+
+// End of Arnoldi step i with ||w|| = t (src/gmres.cpp:226-262): h_{i+1,i} = t,
+// breakdown test, earlier rotations on column i, new rotation, estimate.
+// col: h_0 .. h_i (the last entries are written); c, s: rotations; rs: entry i
+// of the right-hand side and the next.  One thread.
+__device__ __forceinline__ void arnoldi_end(GmresCtl* ctl, int i, double t, double* col, double* c, double* s, double* rs,
+                                            double* hist) {
+    col[i + 1] = t;
+    if (t <= 1e-16) {
+        ctl->breakdown = 1;
+        ctl->cycle_active = 0;
+        return;
+    }
+    ctl->inv = 1.0 / t;
+    for (int k = 1; k <= i; ++k) {
+        const int k1 = k - 1;
+        const double tk = col[k1];
+        col[k1] = c[k1] * tk + s[k1] * col[k];
+        col[k] = -s[k1] * tk + c[k1] * col[k];
+    }
+    const double a = col[i], b = col[i + 1];
+    double gam = std::sqrt(a * a + b * b);
+    if (gam == 0.0) gam = 1e-16;
+    c[i] = col[i] / gam;
+    s[i] = col[i + 1] / gam;
+    rs[1] = -s[i] * rs[0];
+    rs[0] = c[i] * rs[0];
+    col[i] = c[i] * col[i] + s[i] * col[i + 1];
+    const double beta = std::fabs(rs[1]);
+    ctl->beta = beta;
+    if (hist && ctl->nhist < ctl->hist_cap) hist[ctl->nhist++] = beta;
+    if (std::isnan(beta)) {
+        ctl->status = 2;
+        ctl->cycle_active = 0;
+    }
+}
+
+__device__ __forceinline__ void post_step(int* word, const GmresCtl* ctl) {
+    __hip_atomic_store(word, kStepDone | ctl->cycle_active, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// What a Gram-Schmidt kernel needs to end its step: the Hessenberg block, the
+// history and the step's word in the host's view.
+struct StepEnd {
+    double* hh;
+    double* hist;
+    int* word;
+};
+
+// Column i and the rotations while a Gram-Schmidt kernel runs: in LDS for
+// m <= kLdsRestart (the chain of rotations is one thread's, at LDS latency),
+// in the Hessenberg block itself beyond.
+constexpr int kLdsRestart = 1024;
+inline size_t col_bytes(int m) { return m <= kLdsRestart ? sizeof(double) * 3 * (m + 2) : 0; }
+
+// The step's end and the next step's gate by one workgroup that holds h_0 ..
+// h_i in s_col (LDS, m <= kLdsRestart) or in the block.  Every thread calls it.
+__device__ __forceinline__ void end_step(GmresCtl* ctl, int i, int m, double t, double* s_col, const StepEnd& e) {
+    double* const col = e.hh + static_cast<long>(i) * (m + 1);
+    double* const c = e.hh + static_cast<long>(m + 1) * m;
+    double* const s = c + m + 1;
+    double* const rs = s + m + 1 + i;
+    const bool lds = m <= kLdsRestart;
+    double* const s_c = s_col + m + 2;
+    double* const s_s = s_c + m + 2;
+    if (lds)
+        for (int k = threadIdx.x; k < i; k += blockDim.x) {
+            s_c[k] = c[k];
+            s_s[k] = s[k];
+        }
     __syncthreads();
     if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int k = 0; k < kMgsThreads / 64; ++k) t += s_part[k];
-        s_total = t;
+        if (lds) {
+            arnoldi_end(ctl, i, t, s_col, s_c, s_s, rs, e.hist);
+            if (!ctl->breakdown) {
+                c[i] = s_c[i];
+                s[i] = s_s[i];
+            }
+        } else {
+            arnoldi_end(ctl, i, t, col, c, s, rs, e.hist);
+        }
+        if (i + 1 < m) step_gate(ctl, i + 1);
+        post_step(e.word, ctl);
     }
     __syncthreads();
-    return s_total;
+    if (lds)
+        for (int k = threadIdx.x; k <= i + 1; k += blockDim.x) col[k] = s_col[k];
 }
 
 template <int R>
 __global__ __launch_bounds__(kMgsThreads) void k_mgs_all(int n, int i, int m, int chunk, const double* __restrict__ vv,
-                                                         double* w, const double* part0, double* pbuf, double* col,
-                                                         double* tnorm, const GmresCtl* ctl, int* err,
-                                                         uint64_t wd_limit) {
-    if (ctl->step_active == 0) return;
+                                                         double* w, const double* part0, int np, double* pbuf, StepEnd end,
+                                                         GmresCtl* ctl, int* err, uint64_t wd_limit) {
+    extern __shared__ double s_col[];  // workgroup 0: column i, then the rotations
+    __shared__ double s_buf[2 * (kMgsThreads / 64)];
     const int nwg = gridDim.x, wg = blockIdx.x;
+    double* const hcol = m <= kLdsRestart ? s_col : end.hh + static_cast<long>(i) * (m + 1);
+    int turn = 0;
+    if (ctl->step_active == 0) {
+        if (wg == 0 && threadIdx.x == 0) post_step(end.word, ctl);
+        return;
+    }
+    if (wg == 0 && threadIdx.x == 0) ctl->ticks_mv += wall_clock64() - ctl->t_mv;
     double* pb = pbuf + static_cast<long>(i & 1) * (m + 1) * nwg;
     double* pnext = pbuf + static_cast<long>((i + 1) & 1) * (m + 1) * nwg;
     for (int j = threadIdx.x; j <= m; j += kMgsThreads)
@@ -187,11 +312,11 @@ __global__ __launch_bounds__(kMgsThreads) void k_mgs_all(int n, int i, int m, in
     double h = 0.0;
     {
         double v = 0.0;
-        for (int k = threadIdx.x; k < kVecBlocks; k += kMgsThreads) v += part0[k];
-        h = block_sum512(v);
+        for (int k = threadIdx.x; k < np; k += kMgsThreads) v += part0[k];
+        h = block_total<kMgsThreads / 64>(v, s_buf, turn);
     }
     for (int j = 0; j <= i; ++j) {
-        if (wg == 0 && threadIdx.x == 0) col[j] = h;
+        if (wg == 0 && threadIdx.x == 0) hcol[j] = h;
         const bool more = j < i;
         double acc = 0.0;
 #pragma unroll
@@ -199,7 +324,7 @@ __global__ __launch_bounds__(kMgsThreads) void k_mgs_all(int n, int i, int m, in
             wr[k] = fma(-h, vn[k], wr[k]);
             acc = more ? fma(vq[k], wr[k], acc) : fma(wr[k], wr[k], acc);
         }
-        const double tot = block_sum512(acc);
+        const double tot = block_total<kMgsThreads / 64>(acc, s_buf, turn);
         double* slot = pb + static_cast<long>(j) * nwg;
         if (threadIdx.x == 0) publish(slot + wg, tot);
         if (j + 1 < i) {
@@ -225,10 +350,9 @@ __global__ __launch_bounds__(kMgsThreads) void k_mgs_all(int n, int i, int m, in
             }
             v = __longlong_as_double(bits);
         }
-        h = block_sum512(v);
+        h = block_total<kMgsThreads / 64>(v, s_buf, turn);
     }
     const double t = std::sqrt(h);
-    if (wg == 0 && threadIdx.x == 0) *tnorm = t;
     const double a = 1.0 / t;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
@@ -236,6 +360,68 @@ __global__ __launch_bounds__(kMgsThreads) void k_mgs_all(int n, int i, int m, in
         if (r < r1) w[r] = t <= 1e-16 ? wr[k] : wr[k] * a;
     }
     if (timed_out && threadIdx.x == 0) atomicOr(err, kErrTimeout);
+    // every workgroup has read the step's flags: all have published their last partial
+    if (wg == 0) end_step(ctl, i, m, t, s_col, end);
+}
+
+// The same for n <= kSmallRows in one workgroup: every reduction stays in it,
+// where the grid's hand-offs cost 3.8 us per term (58 us per step on 2D Poisson
+// 64^2).  Basis vectors are requested two terms ahead.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallRows = 8 * kSmallThreads;
+
+template <int R>
+__global__ __launch_bounds__(kSmallThreads) void k_mgs_small(int n, int i, int m, const double* __restrict__ vv, double* w,
+                                                             const double* part0, int np, StepEnd end, GmresCtl* ctl) {
+    extern __shared__ double s_col[];
+    __shared__ double s_buf[2 * (kSmallThreads / 64)];
+    double* const hcol = m <= kLdsRestart ? s_col : end.hh + static_cast<long>(i) * (m + 1);
+    int turn = 0;
+    if (ctl->step_active == 0) {
+        if (threadIdx.x == 0) post_step(end.word, ctl);
+        return;
+    }
+    if (threadIdx.x == 0) ctl->ticks_mv += wall_clock64() - ctl->t_mv;
+    double wr[R], vn[R], vq[R], vp[R];
+    auto fetch = [&](int j, double* v) {
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int r = threadIdx.x + k * kSmallThreads;
+            v[k] = r < n && j <= i ? vv[static_cast<long>(j) * n + r] : 0.0;
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int r = threadIdx.x + k * kSmallThreads;
+        wr[k] = r < n ? w[r] : 0.0;
+    }
+    fetch(0, vn);
+    fetch(1, vq);
+    double v = 0.0;
+    for (int k = threadIdx.x; k < np; k += kSmallThreads) v += part0[k];
+    double h = block_total<kSmallThreads / 64>(v, s_buf, turn);
+    for (int j = 0; j <= i; ++j) {
+        fetch(j + 2, vp);
+        if (threadIdx.x == 0) hcol[j] = h;
+        const bool more = j < i;
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            wr[k] = fma(-h, vn[k], wr[k]);
+            acc = more ? fma(vq[k], wr[k], acc) : fma(wr[k], wr[k], acc);
+            vn[k] = vq[k];
+            vq[k] = vp[k];
+        }
+        h = block_total<kSmallThreads / 64>(acc, s_buf, turn);
+    }
+    const double t = std::sqrt(h);
+    const double a = 1.0 / t;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int r = threadIdx.x + k * kSmallThreads;
+        if (r < n) w[r] = t <= 1e-16 ? wr[k] : wr[k] * a;
+    }
+    end_step(ctl, i, m, t, s_col, end);
 }
 
 __global__ void k_fill_pending(long n, uint64_t* p) {
@@ -252,9 +438,10 @@ __global__ __launch_bounds__(kVecThreads) void k_scale(int n, double* v, const G
 }
 
 // Start of a cycle (src/gmres.cpp:185-198).
-__global__ void k_cycle_begin(GmresCtl* ctl, const double* part, double* rs) {
-    const double beta = std::sqrt(sum_partials(part));
+__global__ void k_cycle_begin(GmresCtl* ctl, const double* part, int np, double* rs) {
+    const double beta = std::sqrt(sum_partials(part, np));
     if (threadIdx.x != 0) return;
+    ctl->ticks_mv += wall_clock64() - ctl->t_mv;
     ctl->beta = beta;
     ctl->i = -1;
     ctl->breakdown = 0;
@@ -269,60 +456,21 @@ __global__ void k_cycle_begin(GmresCtl* ctl, const double* part, double* rs) {
     ctl->cycle_active = 1;
 }
 
-// Loop condition of the Krylov loop (src/gmres.cpp:199) for step i.
-__global__ void k_step_gate(GmresCtl* ctl, int i) {
-    if (ctl->cycle_active && ctl->beta > ctl->tol) {
-        const int before = ctl->its++;
-        if (before < ctl->maxits) {
-            ctl->step_active = 1;
-            ctl->i = i;
-            return;
-        }
-    }
-    ctl->step_active = 0;
-    ctl->cycle_active = 0;
+// The gate of step i on its own: a cycle's first step (after v_0 is scaled;
+// no word), and in the per-term path the step's end as the host sees it.
+__global__ void k_step_gate(GmresCtl* ctl, int i, int m, int* word) {
+    if (i < m) step_gate(ctl, i);
+    if (word) post_step(word, ctl);
 }
 
-// End of an Arnoldi step (src/gmres.cpp:226-262): h_{i+1,i} = ||w||,
-// breakdown test, earlier rotations on column i, new rotation, estimate.
-__global__ void k_arnoldi_finish(GmresCtl* ctl, const double* part, const double* tnorm, double* hh, double* hist) {
+// End of an Arnoldi step of the per-term path: ||w|| from the partials.
+__global__ void k_arnoldi_finish(GmresCtl* ctl, const double* part, int np, int m, StepEnd end) {
     if (ctl->step_active == 0) return;
-    const double t = tnorm ? *tnorm : std::sqrt(sum_partials(part));
+    const double t = std::sqrt(sum_partials(part, np));
     if (threadIdx.x != 0) return;
-    const int im = ctl->im, im1 = im + 1;
-    const int i = ctl->i, i1 = i + 1;
-    double* col = hh + static_cast<long>(i) * im1;
-    double* c = hh + static_cast<long>(im1) * im;
-    double* s = c + im1;
-    double* rs = s + im1;
-    col[i1] = t;
-    if (t <= 1e-16) {
-        ctl->breakdown = 1;
-        ctl->cycle_active = 0;
-        return;
-    }
-    ctl->inv = 1.0 / t;
-    for (int k = 1; k <= i; ++k) {
-        const int k1 = k - 1;
-        const double tk = col[k1];
-        col[k1] = c[k1] * tk + s[k1] * col[k];
-        col[k] = -s[k1] * tk + c[k1] * col[k];
-    }
-    const double a = col[i], b = col[i1];
-    double gam = std::sqrt(a * a + b * b);
-    if (gam == 0.0) gam = 1e-16;
-    c[i] = col[i] / gam;
-    s[i] = col[i1] / gam;
-    rs[i1] = -s[i] * rs[i];
-    rs[i] = c[i] * rs[i];
-    col[i] = c[i] * col[i] + s[i] * col[i1];
-    const double beta = std::fabs(rs[i1]);
-    ctl->beta = beta;
-    if (hist && ctl->nhist < ctl->hist_cap) hist[ctl->nhist++] = beta;
-    if (std::isnan(beta)) {
-        ctl->status = 2;
-        ctl->cycle_active = 0;
-    }
+    const int i = ctl->i;
+    double* c = end.hh + static_cast<long>(m + 1) * m;
+    arnoldi_end(ctl, i, t, end.hh + static_cast<long>(i) * (m + 1), c, c + m + 1, c + 2 * (m + 1) + i, end.hist);
 }
 
 // Upper-triangular solve for the step coefficients (src/gmres.cpp:265-272).
@@ -367,8 +515,8 @@ __global__ void k_check_cols(int n, long nnz, const int* __restrict__ ci, int* b
     }
 }
 
-__global__ void k_sqrt_sum(const double* part, double* out) {
-    const double v = std::sqrt(sum_partials(part));
+__global__ void k_sqrt_sum(const double* part, int np, double* out) {
+    const double v = std::sqrt(sum_partials(part, np));
     if (threadIdx.x == 0) *out = v;
 }
 
@@ -381,16 +529,12 @@ struct lljbash::PreconditionedGmres::Ext {
     pilu::DevBuf<pilu::GmresCtl> ctl;
     pilu::DevBuf<int> arp, aci;
     pilu::DevBuf<double> aval, rhs, sol;
-    pilu::GmresCtl* snap = nullptr;  // pinned host snapshots (2 slots)
-    hipEvent_t snap_ev[2] = {nullptr, nullptr};
-    std::vector<hipEvent_t> tev;     // timing events (pairs)
+    int* words = nullptr;            // pinned: the words of a step (2 slots)
     int hist_len = 0;
     double true_res = -1.0;
     std::vector<double> hv, hz;      // host vectors of a host-side preconditioner
     ~Ext() {
-        if (snap) (void)hipHostFree(snap);
-        for (auto& e : snap_ev) if (e) (void)hipEventDestroy(e);
-        for (auto& e : tev) (void)hipEventDestroy(e);
+        if (words) (void)hipHostFree(words);
     }
 };
 
@@ -400,22 +544,31 @@ namespace {
 
 using GExt = PreconditionedGmres::Ext;
 
-template <int G>
-void spmv_g(hipStream_t s, int n, const int* rp, const int* ci, const double* val, double alpha, const double* x,
-            double beta, const double* yin, double* y, const double* dotv, bool nrm, double* part, const int* gate) {
-    pilu::k_spmv<G><<<pilu::kVecBlocks, pilu::kVecThreads, 0, s>>>(n, rp, ci, val, alpha, x, beta, yin, y, dotv,
-                                                                  nrm, part, gate);
+// Blocks of the reducing vector kernels over n rows, `per` rows a block.
+inline int vec_blocks(long n, int per) {
+    return static_cast<int>(std::max<long>(1, std::min<long>((n + per - 1) / per, pilu::kVecBlocks)));
 }
 
-void spmv(int lanes, hipStream_t s, int n, const int* rp, const int* ci, const double* val, double alpha,
-          const double* x, double beta, const double* yin, double* y, const double* dotv, bool nrm, double* part,
-          const int* gate) {
+template <int G>
+int spmv_g(hipStream_t s, int n, const int* rp, const int* ci, const double* val, double alpha, const double* x,
+           double beta, const double* yin, double* y, const double* dotv, bool nrm, double* part, const int* gate,
+           pilu::GmresCtl* clock) {
+    const int blocks = vec_blocks(n, pilu::kVecThreads / G);
+    pilu::k_spmv<G><<<blocks, pilu::kVecThreads, 0, s>>>(n, rp, ci, val, alpha, x, beta, yin, y, dotv, nrm, part, gate,
+                                                         clock);
+    return blocks;
+}
+
+// Returns the number of partials.
+int spmv(int lanes, hipStream_t s, int n, const int* rp, const int* ci, const double* val, double alpha,
+         const double* x, double beta, const double* yin, double* y, const double* dotv, bool nrm, double* part,
+         const int* gate, pilu::GmresCtl* clock) {
     switch (lanes) {
-        case 4: spmv_g<4>(s, n, rp, ci, val, alpha, x, beta, yin, y, dotv, nrm, part, gate); break;
-        case 8: spmv_g<8>(s, n, rp, ci, val, alpha, x, beta, yin, y, dotv, nrm, part, gate); break;
-        case 16: spmv_g<16>(s, n, rp, ci, val, alpha, x, beta, yin, y, dotv, nrm, part, gate); break;
-        case 32: spmv_g<32>(s, n, rp, ci, val, alpha, x, beta, yin, y, dotv, nrm, part, gate); break;
-        default: spmv_g<64>(s, n, rp, ci, val, alpha, x, beta, yin, y, dotv, nrm, part, gate); break;
+        case 4: return spmv_g<4>(s, n, rp, ci, val, alpha, x, beta, yin, y, dotv, nrm, part, gate, clock);
+        case 8: return spmv_g<8>(s, n, rp, ci, val, alpha, x, beta, yin, y, dotv, nrm, part, gate, clock);
+        case 16: return spmv_g<16>(s, n, rp, ci, val, alpha, x, beta, yin, y, dotv, nrm, part, gate, clock);
+        case 32: return spmv_g<32>(s, n, rp, ci, val, alpha, x, beta, yin, y, dotv, nrm, part, gate, clock);
+        default: return spmv_g<64>(s, n, rp, ci, val, alpha, x, beta, yin, y, dotv, nrm, part, gate, clock);
     }
 }
 
@@ -429,16 +582,17 @@ struct MgsPlan {
 };
 
 template <int R>
-bool mgs_fits(int nwg) {
+bool mgs_fits(int nwg, size_t lds) {
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(pilu::k_mgs_all<R>),
-                                                     pilu::kMgsThreads, 0) != hipSuccess)
+                                                     pilu::kMgsThreads, lds) != hipSuccess)
         return false;
     return per_cu >= 1 && nwg <= pilu::kMgsThreads;
 }
 
-MgsPlan plan_mgs(int n) {
+MgsPlan plan_mgs(int n, int m) {
     MgsPlan p;
+    const size_t lds = pilu::col_bytes(m);
     static int cus = -1;
     if (cus < 0) {
         int dev = 0;
@@ -452,11 +606,11 @@ MgsPlan plan_mgs(int n) {
     if (r * pilu::kMgsThreads < chunk) return p;
     bool ok = false;
     switch (r) {
-        case 1: ok = mgs_fits<1>(cus); break;
-        case 2: ok = mgs_fits<2>(cus); break;
-        case 4: ok = mgs_fits<4>(cus); break;
-        case 8: ok = mgs_fits<8>(cus); break;
-        default: ok = mgs_fits<16>(cus); break;
+        case 1: ok = mgs_fits<1>(cus, lds); break;
+        case 2: ok = mgs_fits<2>(cus, lds); break;
+        case 4: ok = mgs_fits<4>(cus, lds); break;
+        case 8: ok = mgs_fits<8>(cus, lds); break;
+        default: ok = mgs_fits<16>(cus, lds); break;
     }
     if (!ok) return p;
     p.nwg = cus;
@@ -467,12 +621,22 @@ MgsPlan plan_mgs(int n) {
 
 template <int R>
 hipError_t launch_mgs_r(const MgsPlan& p, hipStream_t s, int n, int i, int m, const double* vv, double* w,
-                        const double* part0, double* pbuf, double* col, double* tnorm, const pilu::GmresCtl* ctl,
-                        int* err, uint64_t wd) {
+                        const double* part0, int np, double* pbuf, pilu::StepEnd end, pilu::GmresCtl* ctl, int* err,
+                        uint64_t wd) {
     int chunk = p.chunk;
-    void* args[] = {&n, &i, &m, &chunk, &vv, &w, &part0, &pbuf, &col, &tnorm, &ctl, &err, &wd};
+    void* args[] = {&n, &i, &m, &chunk, &vv, &w, &part0, &np, &pbuf, &end, &ctl, &err, &wd};
     return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(pilu::k_mgs_all<R>), dim3(p.nwg),
-                                      dim3(pilu::kMgsThreads), args, 0, s);
+                                      dim3(pilu::kMgsThreads), args, pilu::col_bytes(m), s);
+}
+
+void launch_mgs_small(hipStream_t s, int n, int i, int m, const double* vv, double* w, const double* part0, int np,
+                      pilu::StepEnd end, pilu::GmresCtl* ctl) {
+    const size_t lds = pilu::col_bytes(m);
+    const int r = (n + pilu::kSmallThreads - 1) / pilu::kSmallThreads;
+    if (r <= 1) pilu::k_mgs_small<1><<<1, pilu::kSmallThreads, lds, s>>>(n, i, m, vv, w, part0, np, end, ctl);
+    else if (r <= 2) pilu::k_mgs_small<2><<<1, pilu::kSmallThreads, lds, s>>>(n, i, m, vv, w, part0, np, end, ctl);
+    else if (r <= 4) pilu::k_mgs_small<4><<<1, pilu::kSmallThreads, lds, s>>>(n, i, m, vv, w, part0, np, end, ctl);
+    else pilu::k_mgs_small<8><<<1, pilu::kSmallThreads, lds, s>>>(n, i, m, vv, w, part0, np, end, ctl);
 }
 
 // Set once the runtime refuses a cooperative launch in this process (it
@@ -483,15 +647,15 @@ std::atomic<bool> g_coop_refused{false};
 // The one-launch Gram-Schmidt; false (error cleared) when the runtime
 // refuses the cooperative launch, so the caller can use the per-term kernels.
 bool launch_mgs_all(const MgsPlan& p, hipStream_t s, int n, int i, int m, const double* vv, double* w,
-                    const double* part0, double* pbuf, double* col, double* tnorm, const pilu::GmresCtl* ctl,
-                    int* err, uint64_t wd) {
+                    const double* part0, int np, double* pbuf, const pilu::StepEnd& end, pilu::GmresCtl* ctl, int* err,
+                    uint64_t wd) {
     hipError_t rc;
     switch (p.r) {
-        case 1: rc = launch_mgs_r<1>(p, s, n, i, m, vv, w, part0, pbuf, col, tnorm, ctl, err, wd); break;
-        case 2: rc = launch_mgs_r<2>(p, s, n, i, m, vv, w, part0, pbuf, col, tnorm, ctl, err, wd); break;
-        case 4: rc = launch_mgs_r<4>(p, s, n, i, m, vv, w, part0, pbuf, col, tnorm, ctl, err, wd); break;
-        case 8: rc = launch_mgs_r<8>(p, s, n, i, m, vv, w, part0, pbuf, col, tnorm, ctl, err, wd); break;
-        default: rc = launch_mgs_r<16>(p, s, n, i, m, vv, w, part0, pbuf, col, tnorm, ctl, err, wd); break;
+        case 1: rc = launch_mgs_r<1>(p, s, n, i, m, vv, w, part0, np, pbuf, end, ctl, err, wd); break;
+        case 2: rc = launch_mgs_r<2>(p, s, n, i, m, vv, w, part0, np, pbuf, end, ctl, err, wd); break;
+        case 4: rc = launch_mgs_r<4>(p, s, n, i, m, vv, w, part0, np, pbuf, end, ctl, err, wd); break;
+        case 8: rc = launch_mgs_r<8>(p, s, n, i, m, vv, w, part0, np, pbuf, end, ctl, err, wd); break;
+        default: rc = launch_mgs_r<16>(p, s, n, i, m, vv, w, part0, np, pbuf, end, ctl, err, wd); break;
     }
     if (rc == hipSuccess) return true;
     (void)hipGetLastError();
@@ -499,10 +663,25 @@ bool launch_mgs_all(const MgsPlan& p, hipStream_t s, int n, int i, int m, const 
     return false;
 }
 
-struct TimedPair {
-    hipEvent_t a, b;
-    int kind;  // 0 = mv, 1 = precon
-};
+// Waits until the step that stores into *word has run; throws if the stream
+// ends or fails without it.
+int wait_step(hipStream_t s, const int* word) {
+    for (unsigned spin = 1;; ++spin) {
+        const int v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+        if (v) return v;
+        if ((spin & 0xfff) == 0) {
+            const hipError_t rc = hipStreamQuery(s);
+            if (rc == hipErrorNotReady) {
+                (void)hipGetLastError();
+                continue;
+            }
+            PILU_HIP(rc);
+            if (const int last = __atomic_load_n(word, __ATOMIC_ACQUIRE)) return last;
+            throw std::runtime_error("GMRES: a step ended without reporting");
+        }
+        __builtin_ia32_pause();
+    }
+}
 
 // precon (used when ilu is null): M^-1 on host vectors, called once per
 // Arnoldi step with the step's basis vector copied to the host.
@@ -530,15 +709,15 @@ std::pair<bool, int> solve_core(GExt* e, IluSolver* ilu, const std::function<voi
     e->ctl.reserve(1);
     e->n = n;
     e->m = m;
-    if (!e->snap) {
-        PILU_HIP(hipHostMalloc(reinterpret_cast<void**>(&e->snap), 2 * sizeof(pilu::GmresCtl)));
-        for (auto& ev : e->snap_ev) PILU_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    }
+    const int vblocks = vec_blocks(n, pilu::kVecThreads);
+    if (!e->words) PILU_HIP(hipHostMalloc(reinterpret_cast<void**>(&e->words), 2 * sizeof(int)));
     const double avg = n > 0 ? static_cast<double>(nnz) / n : 1.0;
     const int lanes = pilu::lanes_for_avg(avg);
-    // One-launch Gram-Schmidt when each of the co-resident workgroups can
-    // keep its rows of w in registers.
-    const MgsPlan mgs = g_coop_refused ? MgsPlan{} : plan_mgs(n);
+    // Gram-Schmidt in one workgroup for the smallest systems, in one
+    // cooperative launch while each workgroup can keep its rows of w in
+    // registers, and a launch per term beyond.
+    const bool small = n > 0 && n <= pilu::kSmallRows;
+    const MgsPlan mgs = small || g_coop_refused ? MgsPlan{} : plan_mgs(n, m);
     double* pbuf = nullptr;
     if (mgs.nwg > 0) {
         e->pbuf.reserve(static_cast<size_t>(2) * (m + 1) * mgs.nwg);
@@ -574,43 +753,24 @@ std::pair<bool, int> solve_core(GExt* e, IluSolver* ilu, const std::function<voi
     double* hh = e->hh.get();
     double* part0 = e->part.get();
     double* part1 = part0 + pilu::kVecBlocks;
-    double* tnorm = part0 + 2 * pilu::kVecBlocks;
     int* mgs_err = e->flags.get() + 1;
     PILU_HIP(hipMemsetAsync(mgs_err, 0, sizeof(int), s));
     const uint64_t wd = pilu::watchdog_ticks(10.0);
-    std::vector<TimedPair> timed;
-    size_t ev_used = 0;
-    auto next_event = [&]() {
-        if (ev_used == e->tev.size()) {
-            hipEvent_t ev;
-            PILU_HIP(hipEventCreate(&ev));
-            e->tev.push_back(ev);
-        }
-        return e->tev[ev_used++];
-    };
-    auto t_begin = [&](int kind) {
-        TimedPair p{next_event(), next_event(), kind};
-        PILU_HIP(hipEventRecord(p.a, s));
-        timed.push_back(p);
-    };
-    auto t_end = [&]() { PILU_HIP(hipEventRecord(timed.back().b, s)); };
-
     const auto wall0 = std::chrono::steady_clock::now();
     bool ok = true;
     int its = 0;
     while (its < prm.max_iterations) {
         // r = rhs - A sol, ||r|| (src/gmres.cpp:181-185)
-        t_begin(0);
-        spmv(lanes, s, n, rp, ci, val, -1.0, sol, 1.0, rhs, vv, nullptr, true, part0, nullptr);
-        t_end();
-        pilu::k_cycle_begin<<<1, pilu::kVecThreads, 0, s>>>(dctl, part0, hh + static_cast<long>(im1) * m + 2 * im1);
+        const int np = spmv(lanes, s, n, rp, ci, val, -1.0, sol, 1.0, rhs, vv, nullptr, true, part0, nullptr, dctl);
+        pilu::k_cycle_begin<<<1, pilu::kVecThreads, 0, s>>>(dctl, part0, np, hh + static_cast<long>(im1) * m + 2 * im1);
         PILU_HIP(hipMemcpyAsync(&h, dctl, sizeof(h), hipMemcpyDeviceToHost, s));
         PILU_HIP(hipStreamSynchronize(s));
         if (h.status == 1) break;  // beta <= tol (src/gmres.cpp:186-188)
         // A NaN residual would make the reference's outer loop spin forever
         // (its inner loop never runs); report failure instead.
         if (std::isnan(h.beta)) { ok = false; break; }
-        pilu::k_scale<<<pilu::kVecBlocks, pilu::kVecThreads, 0, s>>>(n, vv, dctl, false);
+        pilu::k_scale<<<vblocks, pilu::kVecThreads, 0, s>>>(n, vv, dctl, false);
+        pilu::k_step_gate<<<1, 1, 0, s>>>(dctl, 0, m, nullptr);
         if (pbuf) {
             const long cnt = static_cast<long>(2) * (m + 1) * mgs.nwg;
             pilu::k_fill_pending<<<grid_for_n(cnt, 256), 256, 0, s>>>(cnt, reinterpret_cast<uint64_t*>(pbuf));
@@ -619,8 +779,9 @@ std::pair<bool, int> solve_core(GExt* e, IluSolver* ilu, const std::function<voi
             double* vi = vv + static_cast<long>(i) * n;
             double* vi1 = vv + static_cast<long>(i + 1) * n;
             double* zi = z + static_cast<long>(i) * n;
-            pilu::k_step_gate<<<1, 1, 0, s>>>(dctl, i);
-            t_begin(1);
+            int* word = e->words + (i & 1);
+            __atomic_store_n(word, 0, __ATOMIC_RELAXED);
+            const pilu::StepEnd end{hh, e->hist.get(), word};
             if (host_precon) {
                 // the step runs only while the cycle is active (the gate the
                 // device kernels read)
@@ -635,39 +796,34 @@ std::pair<bool, int> solve_core(GExt* e, IluSolver* ilu, const std::function<voi
             } else {
                 pilu::ilu_apply(ie, vi, zi, step_gate);
             }
-            t_end();
-            t_begin(0);
-            spmv(lanes, s, n, rp, ci, val, 1.0, zi, 0.0, nullptr, vi1, vv, false, part0, step_gate);
-            t_end();
+            const int npi = spmv(lanes, s, n, rp, ci, val, 1.0, zi, 0.0, nullptr, vi1, vv, false, part0, step_gate, dctl);
             // a refused cooperative launch switches this and later steps to
             // the per-term kernels
-            if (pbuf && !launch_mgs_all(mgs, s, n, i, m, vv, vi1, part0, pbuf, hh + static_cast<long>(i) * im1,
-                                        tnorm, dctl, mgs_err, wd))
+            if (pbuf && !launch_mgs_all(mgs, s, n, i, m, vv, vi1, part0, npi, pbuf, end, dctl, mgs_err, wd))
                 pbuf = nullptr;
-            if (pbuf) {
-                pilu::k_arnoldi_finish<<<1, pilu::kVecThreads, 0, s>>>(dctl, nullptr, tnorm, hh, e->hist.get());
-            } else {
+            if (small) {
+                launch_mgs_small(s, n, i, m, vv, vi1, part0, npi, end, dctl);
+            } else if (!pbuf) {
                 double* pin = part0;
                 double* pout = part1;
+                int np_in = npi;
                 for (int j = 0; j <= i; ++j) {
                     const double* vnext = j < i ? vv + static_cast<long>(j + 1) * n : nullptr;
-                    pilu::k_mgs<<<pilu::kVecBlocks, pilu::kVecThreads, 0, s>>>(
-                        n, vv + static_cast<long>(j) * n, vi1, vnext, pin, pout, hh + static_cast<long>(i) * im1 + j,
-                        step_gate);
+                    pilu::k_mgs<<<vblocks, pilu::kVecThreads, 0, s>>>(
+                        n, vv + static_cast<long>(j) * n, vi1, vnext, pin, np_in, pout,
+                        hh + static_cast<long>(i) * im1 + j, step_gate, j == 0 ? dctl : nullptr);
                     std::swap(pin, pout);
+                    np_in = vblocks;
                 }
-                pilu::k_arnoldi_finish<<<1, pilu::kVecThreads, 0, s>>>(dctl, pin, nullptr, hh, e->hist.get());
-                pilu::k_scale<<<pilu::kVecBlocks, pilu::kVecThreads, 0, s>>>(n, vi1, dctl, true);
+                pilu::k_arnoldi_finish<<<1, pilu::kVecThreads, 0, s>>>(dctl, pin, np_in, m, end);
+                pilu::k_scale<<<vblocks, pilu::kVecThreads, 0, s>>>(n, vi1, dctl, true);
+                pilu::k_step_gate<<<1, 1, 0, s>>>(dctl, i + 1, m, word);
             }
-            PILU_HIP(hipMemcpyAsync(&e->snap[i & 1], dctl, sizeof(h), hipMemcpyDeviceToHost, s));
-            PILU_HIP(hipEventRecord(e->snap_ev[i & 1], s));
-            if (i >= 1) {
-                PILU_HIP(hipEventSynchronize(e->snap_ev[(i - 1) & 1]));
-                if (!e->snap[(i - 1) & 1].cycle_active) break;
-            }
+            PILU_HIP(hipGetLastError());
+            if (i >= 1 && !(wait_step(s, e->words + ((i - 1) & 1)) & 1)) break;
         }
         pilu::k_backsolve<<<1, 64, 0, s>>>(dctl, hh);
-        pilu::k_update<<<pilu::kVecBlocks, pilu::kVecThreads, 0, s>>>(n, z, dctl, hh, sol);
+        pilu::k_update<<<vblocks, pilu::kVecThreads, 0, s>>>(n, z, dctl, hh, sol);
         PILU_HIP(hipGetLastError());
         PILU_HIP(hipMemcpyAsync(&h, dctl, sizeof(h), hipMemcpyDeviceToHost, s));
         PILU_HIP(hipStreamSynchronize(s));
@@ -678,8 +834,9 @@ std::pair<bool, int> solve_core(GExt* e, IluSolver* ilu, const std::function<voi
     }
     its = h.its;
     // FP64 true residual of the returned iterate (reported, not used).
-    spmv(lanes, s, n, rp, ci, val, -1.0, sol, 1.0, rhs, e->scratch.get(), nullptr, true, part0, nullptr);
-    pilu::k_sqrt_sum<<<1, pilu::kVecThreads, 0, s>>>(part0, part1);
+    const int np = spmv(lanes, s, n, rp, ci, val, -1.0, sol, 1.0, rhs, e->scratch.get(), nullptr, true, part0, nullptr,
+                        nullptr);
+    pilu::k_sqrt_sum<<<1, pilu::kVecThreads, 0, s>>>(part0, np, part1);
     PILU_HIP(hipMemcpyAsync(&e->true_res, part1, sizeof(double), hipMemcpyDeviceToHost, s));
     if (ie) pilu::check_sweep_errors(ie);
     if (mgs.nwg > 0) {  // cooperative launches may have run (before a refusal too)
@@ -689,13 +846,9 @@ std::pair<bool, int> solve_core(GExt* e, IluSolver* ilu, const std::function<voi
         if (werr & pilu::kErrTimeout) throw std::runtime_error("GMRES: Gram-Schmidt reduction wait timed out (watchdog)");
     }
     st.total_fgmr_time += std::chrono::duration<double>(std::chrono::steady_clock::now() - wall0).count();
-    for (const auto& p : timed) {
-        float ms = 0.f;
-        if (hipEventElapsedTime(&ms, p.a, p.b) == hipSuccess) {
-            if (p.kind == 0) st.total_mv_time += ms * 1e-3;
-            else st.total_precon_time += ms * 1e-3;
-        }
-    }
+    const double tick = 1.0 / static_cast<double>(pilu::watchdog_ticks(1.0));
+    st.total_mv_time += static_cast<double>(h.ticks_mv) * tick;
+    st.total_precon_time += static_cast<double>(h.ticks_precon) * tick;
     e->hist_len = h.nhist;
     return {ok, its};
 }

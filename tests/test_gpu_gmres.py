@@ -206,3 +206,25 @@ def test_gmres_with_level_walk_sweeps_matches_level_sweeps(oracle):
     fac, dg, _ = oracle.ilu_factorize(o[0], o[1], o[3])
     ok_o, its_o, _, _ = oracle.gmres((rp0, ci0, va0), b, tol, 40, 400, factors=(o[0], o[1], dg, fac))
     assert ok_o and abs(runs[1][0] - its_o) <= 1
+
+
+@pytest.mark.parametrize("n,m", [(70, 12), (1024, 12), (1025, 1), (1025, 1100), (2049, 12), (8192, 12), (8193, 12),
+                                 (8193, 1100)])
+def test_gram_schmidt_forms_match_oracle(oracle, n, m):
+    """Sizes at the edges of the one-workgroup Gram-Schmidt (1024 rows a register,
+    8192 in all) and restarts whose column stays in LDS (up to 1024) or not.  The
+    estimates agree to the rounding of a sum (n eps) times the growth of the
+    recurrence; 1e-6 as for the other histories."""
+    a = gen.random_banded(n, 8, 40, seed=n)
+    b = gen.rhs_uniform(n, seed=2)
+    tol = 1e-9 * np.linalg.norm(b)
+    o, (ok_o, its_o, x_o, hist_o) = oracle_run(oracle, a, 0, b, tol, m, 60)
+    g = gmres(solver_for(o[0], o[1], o[3]), tol, m, 60)
+    x = np.zeros(n)
+    ok, its = g.Solve(P.HostCsr.from_csr(a), b, x)
+    assert ok == ok_o and abs(its - its_o) <= 1
+    hist = g.ResidualHistory()
+    k = min(hist.size, hist_o.size)
+    assert k > 0 and np.allclose(hist[:k], hist_o[:k], rtol=1e-6)
+    st = g.stat()
+    assert 0 < st.total_mv_time + st.total_precon_time <= st.total_fgmr_time
