@@ -122,6 +122,7 @@ __device__ __forceinline__ void levels_body(int n, const int* __restrict__ rp, c
     bool head = G == 1;
     int pub = -1;   // this lane's level once known (read by later lanes of the wave)
     int nl_max = 0; // most in-wave dependencies of a lane of the wave
+    bool chain = false;  // (uniform) the wave's only in-wave dependencies are on the lane before
     if constexpr (G == 1) {
         const long k0 = k - lane;  // schedule position of the wave's first row
         int nl = 0;
@@ -148,6 +149,7 @@ __device__ __forceinline__ void levels_body(int n, const int* __restrict__ rp, c
             }
         }
         e = e + kLevE < end ? e + kLevE : end;
+        chain = __ballot(nl > 1 || (nl == 1 && hl[0] != lane - 1)) == 0;
         for (int off = 1; off < 64; off <<= 1) {
             const int o = __shfl_xor(nl, off, 64);
             nl = o > nl ? o : nl;
@@ -191,9 +193,32 @@ __device__ __forceinline__ void levels_body(int n, const int* __restrict__ rp, c
             }
         }
         if constexpr (G == 1) {
+            // A chain (level = max(own, level of the lane before + 1)) is a
+            // segmented maximum of level - lane over the wave: six steps,
+            // where the passes below take one per row of the chain.
+            if (chain) {
+                constexpr int kWaiting = INT_MAX - 256;
+                const bool ready = !done && !head && e >= end;
+                int key = (done ? pub : ready ? lv : INT_MAX - 64) - lane;
+                int first = done || hl[0] < 0;
+#pragma unroll
+                for (int off = 1; off < 64; off <<= 1) {
+                    const int o = __shfl_up(key, off, 64), of = __shfl_up(first, off, 64);
+                    if (lane >= off && !first) {
+                        key = o > key ? o : key;
+                        first = of;
+                    }
+                }
+                if (!done && key < kWaiting) {
+                    pub = key + lane;
+                    publish_int(level + row, pub);
+                    top = pub > top ? pub : top;
+                    done = true;
+                }
+            }
             // in-wave dependencies from the solving lanes' registers, while
             // some lane of the wave finishes (at most 64 passes)
-            for (int it = 0; it < 64; ++it) {
+            for (int it = 0; it < 64 && !chain; ++it) {
                 bool fin = false;
 #pragma unroll
                 for (int q = 0; q < kLevE; ++q) {

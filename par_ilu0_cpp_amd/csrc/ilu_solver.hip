@@ -1694,14 +1694,35 @@ void sweep_lv_one(Ext* e, const T* val, const double* b, double* out, double* re
 constexpr int kAutoAfter = 2;
 
 // Distinct positive offsets row - column of L's entries in tab (0: free);
-// *over is set when there are more than kOffsets.
+// *over is set when there are more than kOffsets.  Each workgroup collects in
+// LDS and adds its few offsets at the end: with every entry looked up in tab
+// itself the lookups serialised on its line (5 ms for 96 x 97 x 5 ILU(1)).
 constexpr int kOffsets = 16;
-__global__ void k_offsets(int n, const int* __restrict__ rp, const int* __restrict__ dg, const int* __restrict__ ci,
-                          int* tab, int* over) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    for (int p = rp[i]; p < dg[i]; ++p) {
-        const int d = i - ci[p];
+constexpr int kOffsetBlocks = 256;
+
+__global__ __launch_bounds__(256) void k_offsets(int n, const int* __restrict__ rp, const int* __restrict__ dg,
+                                                 const int* __restrict__ ci, int* tab, int* over) {
+    __shared__ int s_tab[kOffsets + 1];
+    if (threadIdx.x <= kOffsets) s_tab[threadIdx.x] = 0;
+    __syncthreads();
+    const int stride = static_cast<int>(gridDim.x * blockDim.x);
+    for (long i = blockIdx.x * blockDim.x + threadIdx.x; i < n && s_tab[kOffsets] == 0; i += stride)
+        for (int p = rp[i]; p < dg[i]; ++p) {
+            const int d = static_cast<int>(i) - ci[p];
+            int k = 0;
+            for (; k < kOffsets; ++k) {
+                int v = s_tab[k];
+                if (v == 0) v = atomicCAS(&s_tab[k], 0, d);
+                if (v == 0 || v == d) break;
+            }
+            if (k == kOffsets) {
+                s_tab[kOffsets] = 1;
+                break;
+            }
+        }
+    __syncthreads();
+    if (threadIdx.x < kOffsets && s_tab[threadIdx.x] != 0) {
+        const int d = s_tab[threadIdx.x];
         int k = 0;
         for (; k < kOffsets; ++k) {
             int v = peek_int(tab + k);
@@ -1710,6 +1731,7 @@ __global__ void k_offsets(int n, const int* __restrict__ rp, const int* __restri
         }
         if (k == kOffsets) *over = 1;
     }
+    if (threadIdx.x == 0 && s_tab[kOffsets]) *over = 1;
 }
 
 // Shape of the natural-order grid whose neighbour offsets are `d` (sorted):
@@ -1769,7 +1791,7 @@ bool build_auto(Ext* e) {
     if (n <= kMaxBlockRows && n <= kAutoNarrow * level_rows) return one_block();
     DevBuf<int> tab(kOffsets + 1);
     k_fill_int<<<1, 64, 0, s>>>(kOffsets + 1, tab.get(), 0);
-    k_offsets<<<grid_for(n, 256), 256, 0, s>>>(n, e->rp.get(), e->dg.get(), e->ci.get(), tab.get(), tab.get() + kOffsets);
+    k_offsets<<<std::min(grid_for(n, 256), kOffsetBlocks), 256, 0, s>>>(n, e->rp.get(), e->dg.get(), e->ci.get(), tab.get(), tab.get() + kOffsets);
     PILU_HIP(hipGetLastError());
     int h[kOffsets + 1];
     PILU_HIP(hipMemcpyAsync(h, tab.get(), sizeof(h), hipMemcpyDeviceToHost, s));

@@ -665,3 +665,24 @@ def test_gmres_with_wave_specialised_sweeps(oracle):
     fac, dg, _ = oracle.ilu_factorize(o[0], o[1], o[3])
     ok_o, its_o, _, _ = oracle.gmres((a.row_ptr, a.col_idx, a.value), b, tol, 50, 1000, factors=(o[0], o[1], dg, fac))
     assert ok_o and abs(runs[1][0] - its_o) <= 1
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 1000])
+@pytest.mark.parametrize("offsets", [(1,), (2,), (1, 2), (1, 64), (1, 63, 65), (1, 70, 71, 72, 73, 74, 75, 76, 77, 78)])
+def test_level_counts_of_banded_patterns(n, offsets):
+    """Depth of both dependency graphs: chains on the row before (resolved as a
+    maximum over the wave), other dependencies inside a wave, and rows with more
+    dependencies than the ones kept in registers; some entries left out."""
+    rng = np.random.default_rng(n + len(offsets))
+    rows = [sorted({i} | {j for o in offsets for j in (i - o, i + o) if 0 <= j < n and rng.random() < 0.9}) for i in range(n)]
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    ci = np.concatenate(rows).astype(np.int32)
+    depth_l, depth_u = np.zeros(n, int), np.zeros(n, int)
+    for i in range(n):
+        depth_l[i] = max((depth_l[j] + 1 for j in rows[i] if j < i), default=0)
+    for i in reversed(range(n)):
+        depth_u[i] = max((depth_u[j] + 1 for j in rows[i] if j > i), default=0)
+    ilu = P.IluSolver(0)
+    ilu.SetMatrix(rp, ci, np.where(ci == np.repeat(np.arange(n), np.diff(rp)), 8.0, -0.25))
+    assert ilu.SetupMatrix() == 0
+    assert ilu.Levels() == (depth_l.max() + 1, depth_u.max() + 1)
