@@ -157,16 +157,33 @@ __device__ __forceinline__ double dpp_row_shl(double v) {
                                                        static_cast<uint32_t>(lo)));
 }
 
+// v of the lane K (16, 32) places up, in the lanes whose bit K is clear (the
+// swap exchanges one operand's lanes with bit K set and the other's without).
+template <int K>
+__device__ __forceinline__ double upper_row(double v) {
+    static_assert(K == 16 || K == 32, "row distance");
+    const unsigned lo = static_cast<unsigned>(__double2loint(v)), hi = static_cast<unsigned>(__double2hiint(v));
+    if constexpr (K == 32) {
+        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        return __hiloint2double(static_cast<int>(h[1]), static_cast<int>(l[1]));
+    } else {
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        return __hiloint2double(static_cast<int>(h[1]), static_cast<int>(l[1]));
+    }
+}
+
 // Sum over G adjacent lanes (G a power of two <= 64), valid in the group's
 // first lane (the others hold partial sums).  Lane 0 adds lane G/2's value,
 // then G/4's, ..., then lane 1's: the addition tree of the xor butterfly,
 // so the result is deterministic for a given G.  Offsets below 16 are DPP
-// row shifts (no LDS traffic); 16 and 32 cross rows through ds_bpermute.
+// row shifts, 16 and 32 row swaps: no LDS traffic.
 // Every lane of the group must be active.
 template <int G>
 __device__ __forceinline__ double group_sum(double v) {
-    if constexpr (G >= 64) v += __shfl_down(v, 32, 64);
-    if constexpr (G >= 32) v += __shfl_down(v, 16, 64);
+    if constexpr (G >= 64) v += upper_row<32>(v);
+    if constexpr (G >= 32) v += upper_row<16>(v);
     if constexpr (G >= 16) v += dpp_row_shl<8>(v);
     if constexpr (G >= 8) v += dpp_row_shl<4>(v);
     if constexpr (G >= 4) v += dpp_row_shl<2>(v);

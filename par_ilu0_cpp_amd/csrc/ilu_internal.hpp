@@ -75,6 +75,22 @@ struct SweepStream {
     int version = -1, g = 0;        // partition (default streams: pattern) and lanes per row it was built for
     long factors = -1;              // factorization its values were gathered from
 };
+
+// Streams of one direction's level walk (ilu_walk.hip), in the waves' step order.
+struct WalkStream {
+    DevBuf<int> perm;                // rows by level, then length
+    DevBuf<int> toff, first, sbase;  // first task per level; first step per task and per wave
+    DevBuf<int2> ctl;                // per step: flags and barriers, first schedule position
+    DevBuf<int> row, brow;           // per step and row slot: row or -1, in the order of the results and of bt
+    DevBuf<unsigned> ref;            // per lane: where the entries' x are
+    DevBuf<double> val64, diag, bt;  // per lane values; per row slot (u_ii, 1 / u_ii); b
+    DevBuf<float> val32;
+    long steps = 0;
+    int g = 0, p = 0, nlev = 0, ntask = 0, per = 0;  // p: entries per lane and step; per: tasks per wave
+    int version = -1;                // pattern it was built for
+    long factors = -1;               // factorization its values were gathered from
+};
+
 // Record streams of the wave-specialised sweep (mode 5) for one direction,
 // built for a partition and a lanes-per-row count.
 struct WsPack {
@@ -155,9 +171,10 @@ struct lljbash::IluSolver::Ext {
     // level-scheduled rows at first, chunk streams after a few applies where
     // the pattern suits them (auto_l / auto_u, decided for auto_pattern and
     // the lanes).
-    bool sweep_default = true, auto_on = false;
+    bool sweep_default = true, auto_on = false, walk_on = false;
     int auto_applies = 0, auto_pattern = -1, auto_lanes[2] = {0, 0};
     pilu::SweepStream auto_l, auto_u;
+    pilu::WalkStream walk_l, walk_u;  // in place of auto_l / auto_u for deep, narrow schedules
     pilu::WsPack ws_l, ws_u;
     // Block partition of the rows: contiguous blocks of blk_rows rows, or
     // tiles of the grid (tile[] != 0, grid[] declared by SetGridShape).

@@ -25,6 +25,7 @@
 #include "ilu_internal.hpp"
 #include "ilu_kernels.hpp"
 #include "ilu_stream.hpp"
+#include "ilu_walk.hpp"
 #include "ilu_sweep_ws.hpp"
 #include "iluk_device.hpp"
 
@@ -808,7 +809,7 @@ void analyse(Ext* e) {
     e->grid[0] = e->grid[1] = e->grid[2] = 0;
     ++e->part_version;
     e->sweep_default = true;
-    e->auto_on = false;
+    e->auto_on = e->walk_on = false;
     e->auto_applies = 0;
     e->auto_pattern = -1;
     e->analysed = true;
@@ -1774,8 +1775,21 @@ bool infer_grid(int n, const std::vector<int>& d, int* shape) {
 // level is about 1 us).
 constexpr int kAutoNarrow = 4, kAutoWide = 40;
 
-bool build_auto(Ext* e) {
-    const int gl = effective_lanes(e, false), gu = effective_lanes(e, true);
+// Waves' worth of rows per level (64 / lanes rows each) up to which the level
+// walk takes the place of level-scheduled rows.  Applies of random bands, walk
+// against rows: 5 waves a level (36k rows, 21 a level, 16 lanes) 1655 and 5727
+// us; 21 (167 a level, 8 lanes) 635 and 782; 25 to 28 (32 lanes) 2013 and 3274,
+// 2304 and 2898; 36 (571 a level, 4 lanes) 321 and 210; 50 (201 a level, 16
+// lanes) 1044 and 848.
+constexpr int kWalkTasks = 28;
+
+bool build_auto_walk(Ext* e, int gl, int gu) {
+    const long levels = std::min(e->nlev_l, e->nlev_u);
+    if (static_cast<long>(e->n) * std::max(gl, gu) > 64L * kWalkTasks * levels) return false;
+    return build_walk(e, false, gl, e->walk_l) && build_walk(e, true, gu, e->walk_u);
+}
+
+bool build_auto_stream(Ext* e, int gl, int gu) {
     if (!stream_width_fits(e, false, gl) || !stream_width_fits(e, true, gu)) return false;
     const int n = e->n;
     hipStream_t s = e->stream;
@@ -1843,17 +1857,19 @@ void count_default_apply(Ext* e) {
     if (e->auto_pattern == e->pattern_version && e->auto_lanes[0] == gl && e->auto_lanes[1] == gu) return;
     if (e->auto_applies++ < kAutoAfter) return;
     SetupScope scope(e->stream);
-    e->auto_on = false;
+    e->auto_on = e->walk_on = false;
     e->auto_pattern = e->pattern_version;
     e->auto_lanes[0] = gl;
     e->auto_lanes[1] = gu;
     try {
-        e->auto_on = build_auto(e);
+        e->auto_on = build_auto_stream(e, gl, gu);
+        if (!e->auto_on) e->walk_on = build_auto_walk(e, gl, gu);
     } catch (const std::runtime_error&) {
         // no acyclic tiles, or no memory for the streams: level-scheduled rows stay
         (void)hipGetLastError();
     }
     e->auto_l.version = e->auto_u.version = e->auto_on ? e->pattern_version : -1;
+    e->walk_l.version = e->walk_u.version = e->walk_on ? e->pattern_version : -1;
 }
 
 // The stream that replaces the level-scheduled sweep of a direction, or null.
@@ -1864,6 +1880,15 @@ const SweepStream* auto_stream(Ext* e, bool upper) {
         return nullptr;
     if (e->factored && st.factors != e->factor_version) gather_stream(e, upper, st);
     return &st;
+}
+
+// The same for the level walk.
+const WalkStream* auto_walk(Ext* e, bool upper) {
+    WalkStream& w = upper ? e->walk_u : e->walk_l;
+    if (!e->sweep_default || !e->walk_on || w.version != e->pattern_version || w.g != effective_lanes(e, upper))
+        return nullptr;
+    if (e->factored && w.factors != e->factor_version) gather_walk(e, upper, w);
+    return &w;
 }
 
 template <typename T, bool UPPER>
@@ -1899,11 +1924,16 @@ void sweep_dispatch(int lanes, Ext* e, const T* val, const double* b, double* ou
         sweep_blk_dispatch<T, UPPER>(lanes, e, val, b, out, reset, gate, ctr);
         return;
     }
-    if (mode == 0)
+    if (mode == 0) {
         if (const SweepStream* st = auto_stream(e, UPPER)) {
             sweep_stream(e, UPPER, *st, b, out, reset, gate, ctr, e->err.get() + kErrSweep);
             return;
         }
+        if (const WalkStream* w = auto_walk(e, UPPER)) {
+            sweep_walk(e, UPPER, *w, b, out, reset, gate);
+            return;
+        }
+    }
     switch (lanes) {
         case 1: sweep_one<1, T, UPPER>(e, val, b, out, reset, gate, ctr); break;
         case 2: sweep_one<2, T, UPPER>(e, val, b, out, reset, gate, ctr); break;
@@ -1987,6 +2017,8 @@ bool run_factor(Ext* e) {
         SweepStream& at = upper ? e->auto_u : e->auto_l;
         if (st.version == e->part_version && st.lds > 0) gather_stream(e, upper, st);
         if (e->sweep_default && at.version == e->pattern_version && at.lds > 0) gather_stream(e, upper, at);
+        WalkStream& w = upper ? e->walk_u : e->walk_l;
+        if (e->sweep_default && e->walk_on && w.version == e->pattern_version) gather_walk(e, upper, w);
     }
     if (ws_current(e, e->ws_l, e->ws_l.g)) gather_ws(e, e->ws_l);
     if (ws_current(e, e->ws_u, e->ws_u.g)) gather_ws(e, e->ws_u);
@@ -2013,7 +2045,7 @@ void show_algorithm(const lljbash::IluSolver* solver) {
 bool flags_in_output(Ext* e, bool upper) {
     const int mode = upper ? e->mode_u : e->mode_l;
     if (mode < 0 || mode > 3) return false;
-    if (mode == 0) return !auto_stream(e, upper);
+    if (mode == 0) return !auto_stream(e, upper) && !auto_walk(e, upper);
     return mode == 1 || !packed_stream(e, upper, pp_lanes(effective_lanes(e, upper)));
 }
 

@@ -171,3 +171,63 @@ def test_default_sweeps_without_a_grid():
         first = ilu.Substitute(b)
         for _ in range(4):
             assert np.array_equal(ilu.Substitute(b), first)
+
+
+def walk_pattern(kind, dominant):
+    rng = np.random.default_rng(11)
+    if kind == "chain":  # one row a level, dependencies both sides of the LDS ring's 16384 rows
+        n = 36000
+        cols = [sorted({i} | ({i - 1} if i and i % 500 else set()) |
+                       {j for j in (i - 16383, i - 16384, i - 16390, i - 30000) if j >= 0 and i % 7 == 0}) for i in range(n)]
+    elif kind == "wide":  # a level wider than the ring allows
+        n = 7000
+        cols = [sorted({i} | ({i - 1} if i > 5000 else set())) for i in range(n)]
+    else:  # levels of a few rows, rows from empty to 300 entries
+        n = {"one": 1, "few": 70, "rows": 9001}[kind]
+        cols = [sorted({i} | {int(j) for j in rng.integers(max(0, i - 400), i + 1, int(rng.integers(0, 300)) if i % 5 else 3)})
+                for i in range(n)]
+    lower = [[c for c in r if c < i] for i, r in enumerate(cols)]
+    upper = [[] for _ in range(n)]
+    for i, r in enumerate(lower):
+        for c in r:
+            upper[c].append(i)
+    rows = [lower[i] + [i] + sorted(upper[i]) for i in range(n)]
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    ci = np.concatenate(rows).astype(np.int32)
+    va = rng.uniform(-1, 1, ci.size) / 64
+    on = ci == np.repeat(np.arange(n), np.diff(rp))
+    va[on] = rng.uniform(1, 2, n) * 2.0 ** rng.integers(-20, 20, n)  # results to infinity and NaN
+    if dominant:
+        va[on] = 1.1 * np.add.reduceat(np.where(on, 0.0, np.abs(va)), rp[:-1]) + 0.5
+    return rp, ci, va
+
+
+@pytest.mark.parametrize("bits", [64, 32])
+@pytest.mark.parametrize("dominant", [True, False])
+@pytest.mark.parametrize("kind,lanes", [("one", 64), ("few", 32), ("rows", 4), ("rows", 8), ("rows", 16), ("rows", 32),
+                                        ("rows", 64), ("chain", 4), ("chain", 64), ("wide", 32)])
+def test_level_walk_keeps_the_bits_of_level_rows(kind, lanes, dominant, bits):
+    """Deep, narrow schedules of a default-shaped solver go to one workgroup
+    after a few applies: the same bits as the level-scheduled rows before, for
+    both triangles, special values, in place, and after a new factorization."""
+    rp, ci, va = walk_pattern(kind, dominant)
+    n = rp.size - 1
+    ilu = factored(rp, ci, va, bits)
+    ilu.SetSweepLanes(lanes, lanes)
+    rng = np.random.default_rng(6)
+    b = rng.uniform(-1, 1, n)
+    odd = b.copy()
+    odd[rng.integers(0, n, max(1, n // 50))] = 0.0
+    odd[n // 2] = np.inf
+    want = [ilu.Substitute(v) for v in (b, odd)]
+    assert not dominant or np.isfinite(want[0]).all()
+    for _ in range(2):
+        for v, w in zip((b, odd), want):
+            assert np.array_equal(ilu.Substitute(v), w, equal_nan=True)
+    y = ilu.Trsv(False, 1.0, b)
+    assert np.array_equal(ilu.Trsv(True, 1.0, y), want[0], equal_nan=True)
+    P.fill_csr(ilu.GetMatrix(), rp, ci, va * 1.25)
+    assert ilu.Factorize() == 0
+    again = ilu.Substitute(b)
+    ilu.SetSweepMode(0, 0, 0)
+    assert np.array_equal(ilu.Substitute(b), again, equal_nan=True)
