@@ -25,7 +25,8 @@ namespace pilu {
 // Device allocation behind DevBuf.  Inside a SetupScope (per host thread)
 // freed blocks are kept and handed out again (best fit, at most twice the
 // request) instead of going back to the driver; the outermost scope's end
-// synchronises its stream and frees them.  All work on such blocks inside a
+// synchronises its stream and frees them.  Blocks freed outside go to a bounded
+// pool that all solvers allocate from.  All work on such blocks inside a
 // scope must be ordered on that one stream.
 void* dev_alloc(size_t bytes);
 void dev_free(void* p, size_t bytes);

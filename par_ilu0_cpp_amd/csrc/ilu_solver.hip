@@ -20,6 +20,7 @@
 #include <memory>
 #include <mutex>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 #include "ilu_internal.hpp"
@@ -46,6 +47,109 @@ struct ScopeCache {
     std::vector<std::pair<void*, size_t>> blocks;
 };
 thread_local ScopeCache g_scope;
+
+// Freed blocks of all solvers.  A driver allocation or free of some hundred
+// MB costs 0.1 to several ms (and now and then tens): a solver for a new
+// 128^3 ILU(1) pattern and the old one's end 27 ms, often 60, of which the
+// kernels are 8.  At most kPoolBytes are kept, the oldest go first; all are
+// given back when the last block in use is freed and before an allocation
+// fails for want of memory.  Like hipFree, a reuse waits for the device:
+// once for all blocks freed since the last time, in the allocation, so that
+// it does not matter which streams or threads used them.
+constexpr size_t kPoolBytes = size_t{4} << 30;
+
+class BlockPool {
+public:
+    void* take(size_t bytes) {
+        int dev = 0;
+        PILU_HIP(hipGetDevice(&dev));
+        std::lock_guard<std::mutex> lock(mu_);
+        size_t at = free_.size();
+        for (size_t i = 0; i < free_.size(); ++i) {
+            const Block& f = free_[i];
+            if (f.dev == dev && f.bytes >= bytes && f.bytes - bytes <= bytes / 4 && (at == free_.size() || f.bytes < free_[at].bytes))
+                at = i;
+        }
+        if (at < free_.size() && free_[at].dirty) {
+            if (hipDeviceSynchronize() == hipSuccess) {
+                for (Block& f : free_)
+                    if (f.dev == dev) f.dirty = false;
+            } else {  // for instance while a stream is captured
+                (void)hipGetLastError();
+                at = free_.size();
+            }
+        }
+        if (at < free_.size()) {
+            const Block f = free_[at];
+            used_.emplace(f.p, f);
+            free_.erase(free_.begin() + static_cast<long>(at));
+            held_ -= f.bytes;
+            return f.p;
+        }
+        void* p = nullptr;
+        hipError_t rc = hipMalloc(&p, bytes);
+        if (rc == hipErrorOutOfMemory && !free_.empty()) {
+            (void)hipGetLastError();
+            trim(0);
+            rc = hipMalloc(&p, bytes);
+        }
+        PILU_HIP(rc);
+        try {
+            used_.emplace(p, Block{p, bytes, dev, false});
+        } catch (...) {
+            (void)hipFree(p);
+            throw;
+        }
+        return p;
+    }
+
+    void give(void* p) noexcept {
+        std::lock_guard<std::mutex> lock(mu_);
+        const auto it = used_.find(p);
+        if (it == used_.end()) {
+            (void)hipFree(p);
+            return;
+        }
+        Block f = it->second;
+        f.dirty = true;
+        used_.erase(it);
+        try {
+            free_.push_back(f);
+            held_ += f.bytes;
+        } catch (...) {
+            (void)hipFree(p);
+        }
+        trim(used_.empty() ? 0 : kPoolBytes);
+    }
+
+private:
+    struct Block {
+        void* p;
+        size_t bytes;
+        int dev;
+        bool dirty;  // freed since the device was last waited for
+    };
+
+    void trim(size_t keep) {
+        size_t n = 0;
+        while (n < free_.size() && held_ > keep) {
+            (void)hipFree(free_[n].p);
+            held_ -= free_[n++].bytes;
+        }
+        free_.erase(free_.begin(), free_.begin() + static_cast<long>(n));
+    }
+
+    std::mutex mu_;
+    std::unordered_map<void*, Block> used_;
+    std::vector<Block> free_;  // oldest first
+    size_t held_ = 0;
+};
+
+// Never destroyed: solvers with static storage are freed through it at exit.
+BlockPool& pool() {
+    static BlockPool* p = new BlockPool;
+    return *p;
+}
 }  // namespace
 
 void* dev_alloc(size_t bytes) {
@@ -65,9 +169,7 @@ void* dev_alloc(size_t bytes) {
             return p;
         }
     }
-    void* p = nullptr;
-    PILU_HIP(hipMalloc(&p, bytes));
-    return p;
+    return pool().take(bytes);
 }
 
 void dev_free(void* p, size_t bytes) {
@@ -76,7 +178,7 @@ void dev_free(void* p, size_t bytes) {
         g_scope.blocks.emplace_back(p, bytes);
         return;
     }
-    (void)hipFree(p);
+    pool().give(p);
 }
 
 SetupScope::SetupScope(hipStream_t s) {
@@ -86,7 +188,7 @@ SetupScope::SetupScope(hipStream_t s) {
 SetupScope::~SetupScope() {
     if (--g_scope.depth > 0 || g_scope.blocks.empty()) return;
     (void)hipStreamSynchronize(g_scope.stream);  // no kernel may still use a block
-    for (auto& b : g_scope.blocks) (void)hipFree(b.first);
+    for (auto& b : g_scope.blocks) pool().give(b.first);
     g_scope.blocks.clear();
 }
 
