@@ -1115,20 +1115,30 @@ __device__ __forceinline__ void guard_pivot(const PivotGuard& pg, double* piv, i
 // Updates to a row entry arrive in ascending-k order, exactly as in the
 // reference; each uses one fma, the contraction the reference's
 // -ffast-math -march=native build applies.  Row i's values are staged in
-// LDS (capacity CAP per group); entries of U(k) are matched into row i by
+// LDS (cap entries per group, the longest row); entries of U(k) are matched into row i by
 // binary search over its sorted columns.  vin holds the values to factor,
 // vout (all kPending on entry) receives the factors, published entry by
 // entry as value-flags; f32 (optional) receives a float copy.
-// err bit 0: a zero pivot was divided by; bit 1: a row exceeded CAP (its
+// err bit 0: a zero pivot was divided by; bit 1: a row exceeded cap (its
 // factors are published as NaN so that dependent rows still finish).
 // omega (optional): per-row diagonal compensation.  Updates u_kj * a_ik that
 // fall outside row i's pattern are summed (lane-strided, then a fixed
 // butterfly) and omega[i] times that sum is added to a_ii before the row is
 // published -- modified ILU with a per-row relaxation factor.  pg: the
 // pivot check above, after the compensation.
+//
+// A row's pivots form a chain, so rows in flight times the time per pivot
+// bounds it.  The next pivot's columns and values (the first kFacAhead per
+// lane) and the bounds of the one after it are requested while a pivot is
+// applied; its columns are matched once, before its values are waited for.
+// Rows of 266 entries and 133 pivots (ILU(2) of a random band, n = 40k):
+// 28.2 -> 16.2 ms, with LDS for the longest row (788 entries: sixteen rows per
+// CU) instead of 2560 entries (four).
 // ---------------------------------------------------------------------
-template <int G, int CAP>
-__global__ __launch_bounds__(kBlock) void k_factor(int n, const int* __restrict__ perm,
+constexpr int kFacAhead = 4;
+
+template <int G>
+__global__ __launch_bounds__(kBlock) void k_factor(int n, int cap, const int* __restrict__ perm,
                                                    const int* __restrict__ rp,
                                                    const int* __restrict__ ci,
                                                    const int* __restrict__ dg,
@@ -1137,8 +1147,7 @@ __global__ __launch_bounds__(kBlock) void k_factor(int n, const int* __restrict_
                                                    const float* __restrict__ omega, const PivotGuard pg) {
     constexpr int R = 64 / G;
     constexpr int GROUPS = kBlock / G;
-    __shared__ int s_col[GROUPS][CAP];
-    __shared__ double s_val[GROUPS][CAP];
+    extern __shared__ double s_rows[];  // the groups' values, then their columns
     const int ticket = take_ticket(ctr);
     const Watchdog wd(wd_limit);
     const int lane = threadIdx.x & 63;
@@ -1148,8 +1157,8 @@ __global__ __launch_bounds__(kBlock) void k_factor(int n, const int* __restrict_
     const int t = lane & (G - 1);
     const long pos = static_cast<long>(ticket) * GROUPS + grp;
     const bool active = pos < n;
-    int* col = s_col[grp];
-    double* val = s_val[grp];
+    double* val = s_rows + grp * cap;
+    int* col = reinterpret_cast<int*>(s_rows + GROUPS * cap) + grp * cap;
     int row = 0, rb = 0, len = 0, ndiag = 0;
     bool overflow = false;
     if (active) {
@@ -1157,7 +1166,7 @@ __global__ __launch_bounds__(kBlock) void k_factor(int n, const int* __restrict_
         rb = rp[row];
         len = rp[row + 1] - rb;
         ndiag = dg[row] - rb;
-        overflow = len > CAP;
+        overflow = len > cap;
         if (!overflow) {
             for (int q = t; q < len; q += G) {
                 col[q] = ci[rb + q];
@@ -1168,9 +1177,70 @@ __global__ __launch_bounds__(kBlock) void k_factor(int n, const int* __restrict_
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    // this lane's part of a pivot row: entries first, first + G, ... < end
+    struct Pivot {
+        int dk, end;              // diagonal position, end of the row
+        int j[kFacAhead];         // columns
+        uint64_t ub, u[kFacAhead];  // u_kk, values; kPending if not there yet
+    };
+    Pivot cur, next;
+    int dk2 = 0, end2 = 0;
+    auto bounds = [&](int q, int& dk, int& end) {
+        if (q < ndiag) {
+            const int c = col[q];
+            dk = dg[c];
+            end = rp[c + 1];
+        }
+    };
+    auto request = [&](int q, Pivot& v) {
+        v.ub = kPending;
+#pragma unroll
+        for (int c = 0; c < kFacAhead; ++c) {
+            v.j[c] = 0;
+            v.u[c] = kPending;
+        }
+        if (q < ndiag) {
+            v.ub = peek_bits(vout + v.dk);
+#pragma unroll
+            for (int c = 0; c < kFacAhead; ++c) {
+                const int e = v.dk + 1 + t + c * G;
+                if (e < v.end) {
+                    v.j[c] = ci[e];
+                    v.u[c] = peek_bits(vout + e);
+                }
+            }
+        }
+    };
+    // slots of the current pivot's columns in row i (-1: outside the pattern)
+    int tgt[kFacAhead];
+    auto match = [&](int p) {
+        int lo[kFacAhead], hi[kFacAhead];
+#pragma unroll
+        for (int c = 0; c < kFacAhead; ++c) {
+            lo[c] = p + 1;
+            hi[c] = cur.dk + 1 + t + c * G < cur.end ? len : p + 1;
+        }
+        for (int w = len - p - 1; w > 0; w >>= 1)  // enough halvings for any of them
+#pragma unroll
+            for (int c = 0; c < kFacAhead; ++c)
+                if (lo[c] < hi[c]) {
+                    const int mid = (lo[c] + hi[c]) >> 1;
+                    if (col[mid] < cur.j[c]) lo[c] = mid + 1;
+                    else hi[c] = mid;
+                }
+#pragma unroll
+        for (int c = 0; c < kFacAhead; ++c) tgt[c] = lo[c] < len && col[lo[c]] == cur.j[c] ? lo[c] : -1;
+    };
     int p = 0;  // next pivot (uniform within the group)
+    bool ahead = false;  // the pivots after p are requested, p is matched
     double dropped = 0.0;  // this lane's share of the fill updates outside the pattern
     bool done = !active;
+    cur.dk = cur.end = next.dk = next.end = 0;
+    if (!overflow) {
+        bounds(0, cur.dk, cur.end);
+        bounds(1, next.dk, next.end);
+        request(0, cur);
+    }
     if (active && overflow) {
         for (int q = t; q < len; q += G) {
             publish(vout + rb + q, __longlong_as_double(kQuietNan));
@@ -1182,17 +1252,36 @@ __global__ __launch_bounds__(kBlock) void k_factor(int n, const int* __restrict_
     while (true) {
         if (!done) {
             while (p < ndiag) {
-                const int k = col[p];
-                const int dk = dg[k];
-                const int ke = rp[k + 1];
-                const uint64_t ub = peek_bits(vout + dk);
-                bool ok = ub != kPending;
-                for (int q = dk + 1 + t; ok && q < ke; q += G) ok = peek_bits(vout + q) != kPending;
+                if (!ahead) {
+                    request(p + 1, next);
+                    bounds(p + 2, dk2, end2);
+                    match(p);
+                    ahead = true;
+                }
+                const int dk = cur.dk, ke = cur.end;
+                if (cur.ub == kPending) cur.ub = peek_bits(vout + dk);
+                bool ok = cur.ub != kPending;
+#pragma unroll
+                for (int c = 0; c < kFacAhead; ++c) {
+                    const int q = dk + 1 + t + c * G;
+                    if (q < ke) {
+                        if (cur.u[c] == kPending) cur.u[c] = peek_bits(vout + q);
+                        ok = ok && cur.u[c] != kPending;
+                    }
+                }
+                for (int q = dk + 1 + t + kFacAhead * G; ok && q < ke; q += G) ok = peek_bits(vout + q) != kPending;
                 if (!group_all<G>(ok)) break;
-                const double ukk = __longlong_as_double(ub);
+                const double ukk = __longlong_as_double(cur.ub);
                 const double lik = val[p] / ukk;
                 if (ukk == 0.0 && t == 0) atomicOr(err, 1);
-                for (int q = dk + 1 + t; q < ke; q += G) {
+#pragma unroll
+                for (int c = 0; c < kFacAhead; ++c)
+                    if (dk + 1 + t + c * G < ke) {
+                        const double u = __longlong_as_double(cur.u[c]);
+                        if (tgt[c] >= 0) val[tgt[c]] = fma(-u, lik, val[tgt[c]]);
+                        else dropped = fma(-u, lik, dropped);
+                    }
+                for (int q = dk + 1 + t + kFacAhead * G; q < ke; q += G) {
                     const int j = ci[q];
                     int lo = p + 1, hi = len;
                     while (lo < hi) {
@@ -1208,6 +1297,10 @@ __global__ __launch_bounds__(kBlock) void k_factor(int n, const int* __restrict_
                 __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
                 ++p;
+                cur = next;
+                next.dk = dk2;
+                next.end = end2;
+                ahead = false;
             }
             if (p < ndiag && group_all<G>(wd.expired())) {
                 if (t == 0) atomicOr(err, kErrTimeout);

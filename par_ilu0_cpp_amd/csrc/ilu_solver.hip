@@ -2069,14 +2069,19 @@ void factor_short_one(Ext* e, float* f32) {
                                                              pivot_guard(e));
 }
 
-template <int G, int CAP>
+// LDS for the longest row only: it decides how many rows a CU holds.
+template <int G>
 void factor_one(Ext* e, float* f32) {
     constexpr int groups = kBlock / G;
     const int grid = grid_for(e->n, groups);
-    k_factor<G, CAP><<<grid, kBlock, 0, e->stream>>>(e->n, e->perm_l.get(), e->rp.get(), e->ci.get(),
-                                                    e->dg.get(), e->vin.get(), e->fac.get(), f32,
-                                                    e->err.get() + kErrFactor, e->ctr.get() + 2,
-                                                    watchdog_ticks(e->watchdog_s), e->omega_ptr, pivot_guard(e));
+    const int cap = e->max_row;
+    const size_t lds = static_cast<size_t>(groups) * cap * (sizeof(double) + sizeof(int));
+    auto kern = k_factor<G>;
+    PILU_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 static_cast<int>(lds)));
+    kern<<<grid, kBlock, lds, e->stream>>>(e->n, cap, e->perm_l.get(), e->rp.get(), e->ci.get(), e->dg.get(),
+                                           e->vin.get(), e->fac.get(), f32, e->err.get() + kErrFactor, e->ctr.get() + 2,
+                                           watchdog_ticks(e->watchdog_s), e->omega_ptr, pivot_guard(e));
 }
 
 // Runs the factorization kernel on e->vin; returns false on a zero pivot.
@@ -2097,10 +2102,10 @@ bool run_factor(Ext* e) {
     // short rows (stencils up to ILU(1) of a 3D 7-point operator): every
     // pivot row fetched at once, one entry per lane
     if (mr <= 32 && e->max_lo <= 8 && e->max_up <= 8) factor_short_one<8, 32, 8>(e, f32);
-    else if (mr <= 32) factor_one<8, 32>(e, f32);
-    else if (mr <= 64) factor_one<16, 64>(e, f32);
-    else if (mr <= 256) factor_one<32, 256>(e, f32);
-    else if (mr <= 2560) factor_one<64, 2560>(e, f32);
+    else if (mr <= 32) factor_one<8>(e, f32);
+    else if (mr <= 64) factor_one<16>(e, f32);
+    else if (mr <= 256) factor_one<32>(e, f32);
+    else if (mr <= 2560) factor_one<64>(e, f32);
     else throw std::runtime_error("row longer than 2560 entries: not supported by the device factorization");
     PILU_HIP(hipGetLastError());
     const int err = read_int(e->err.get() + kErrFactor, s);

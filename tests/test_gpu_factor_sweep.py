@@ -686,3 +686,20 @@ def test_level_counts_of_banded_patterns(n, offsets):
     ilu.SetMatrix(rp, ci, np.where(ci == np.repeat(np.arange(n), np.diff(rp)), 8.0, -0.25))
     assert ilu.SetupMatrix() == 0
     assert ilu.Levels() == (depth_l.max() + 1, depth_u.max() + 1)
+
+
+@pytest.mark.parametrize("n", [33, 64, 65, 130, 200, 256, 257, 300, 520])
+def test_pivot_rows_longer_than_what_is_requested_ahead(oracle, n):
+    """Dense blocks of n rows (every row a pivot of all later ones), one with its
+    last row thinned out: pivot rows of up to, and more than, four entries per
+    lane in each of the lane counts."""
+    rp = np.arange(0, n * n + 1, n, dtype=np.int32)
+    ci = np.tile(np.arange(n, dtype=np.int32), n)
+    keep = np.ones(n * n, bool)
+    keep[(n - 1) * n : n * n - 1 : 3] = False
+    rp = np.concatenate([[0], np.cumsum(keep.reshape(n, n).sum(1))]).astype(np.int32)
+    ci = ci[keep]
+    va = dominant_values(rp, ci, seed=n)
+    ilu = factored(rp, ci, va)
+    ofac, dg, z = oracle.ilu_factorize(rp, ci, va)
+    assert z == 0 and np.array_equal(host_factors(ilu, ci.size), ofac)
