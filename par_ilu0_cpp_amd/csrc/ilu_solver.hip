@@ -2058,11 +2058,25 @@ PivotGuard pivot_guard(Ext* e) {
     return PivotGuard{e->pivot_mode, e->pivot_tiny, e->pivot_repl, e->err.get() + kErrPivotRow};
 }
 
+// Rows in flight that only wait slow down the few that the level chain is
+// waiting for: where a level is narrow, at most kFactorPerCu workgroups run on
+// a CU (16384 rows on the GPU).  128^3 ILU(1), 2749 rows a level: 3.44 ms with
+// as many as fit, 2.72 with two, 3.20 with one; 96 x 97 x 5 ILU(1): 2.35, 1.78
+// and 1.68; 2D Poisson 64^2 the same.  Levels of more than a quarter of those
+// rows take what fits.
+constexpr int kFactorPerCu = 2;
+constexpr long kFactorNarrow = 4096;
+
 template <int G, int CAP, int P>
 void factor_short_one(Ext* e, float* f32) {
     constexpr int groups = kBlock / G;
     const int grid = grid_for(e->n, groups);
-    k_factor_short<G, CAP, P><<<grid, kBlock, 0, e->stream>>>(e->n, e->perm_l.get(), e->rp.get(), e->ci.get(),
+    auto kern = k_factor_short<G, CAP, P>;
+    constexpr int rows_lds = groups * (CAP * (sizeof(int) + sizeof(double)) + P * sizeof(double2));
+    constexpr int limit = 160 * 1024 / (kFactorPerCu + 1) + 1024 - rows_lds;  // LDS that leaves no room for another
+    const int lds = e->n <= kFactorNarrow * e->nlev_l ? limit : 0;
+    PILU_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, limit));
+    kern<<<grid, kBlock, lds, e->stream>>>(e->n, e->perm_l.get(), e->rp.get(), e->ci.get(),
                                                              e->dg.get(), e->vin.get(), e->fac.get(), f32,
                                                              e->err.get() + kErrFactor, e->ctr.get() + 2,
                                                              watchdog_ticks(e->watchdog_s), e->omega_ptr,

@@ -703,3 +703,19 @@ def test_pivot_rows_longer_than_what_is_requested_ahead(oracle, n):
     ilu = factored(rp, ci, va)
     ofac, dg, z = oracle.ilu_factorize(rp, ci, va)
     assert z == 0 and np.array_equal(host_factors(ilu, ci.size), ofac)
+
+
+@pytest.mark.parametrize("levels", [2, 3, 5])
+def test_short_row_factors_of_wide_and_narrow_levels(oracle, levels):
+    """Short rows in levels of more and of fewer rows than the line up to which
+    the rows in flight are limited (4096 a level)."""
+    width = 12000 // levels
+    n = width * levels
+    rows = [sorted({i} | {j for j in (i - width, i - width + 1, i + width) if 0 <= j < n and j // width != i // width})
+            for i in range(n)]
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    ci = np.concatenate(rows).astype(np.int32)
+    va = dominant_values(rp, ci, seed=levels)
+    ilu = factored(rp, ci, va)
+    ofac, dg, z = oracle.ilu_factorize(rp, ci, va)
+    assert z == 0 and np.array_equal(host_factors(ilu, ci.size), ofac)
