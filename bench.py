@@ -85,7 +85,7 @@ def parse():
     return p.parse_args()
 
 
-SWEEP_KERNELS = {0: "k_sweep", 1: "k_sweep_blk", 2: "k_sweep_pp (level barriers)", 3: "k_sweep_pp (LDS value-flags)",
+SWEEP_KERNELS = {0: "k_sweep", 1: "k_sweep_blk", 2: "k_sweep_st (chunk streams)", 3: "k_sweep_st (chunk streams)",
                  4: "k_sweep_lv (one workgroup, level barriers)", 5: "k_sweep_ws (wave-specialised)"}
 MILU_OMEGA = 0.98  # the constant modified-ILU relaxation of the fp32-milu form
 

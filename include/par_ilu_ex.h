@@ -86,7 +86,8 @@ int IluSolverAutotuneEx(IluSolverHdl hdl, int reps, double* table, int cap);
 /* Explicit sweep algorithm per direction (0 level rows, 1 block-local over
  * contiguous blocks of blk_rows rows, 2 block-local over packed factors,
  * software-pipelined, with a workgroup barrier per local level, 3 the same
- * with the block's x as LDS value-flags and no barriers, 4 one workgroup
+ * with the block's x as LDS value-flags and no barriers (2 and 3 run over chunk
+ * streams where every row has at most one entry per lane), 4 one workgroup
  * walking the level schedule with a barrier per level, for deep schedules
  * with few rows per level, 5 block-local with one solver, one record-stream
  * loader and one importer wave per block, 1-16 lanes per row; blk_rows is

@@ -161,16 +161,17 @@ struct lljbash::IluSolver::Ext {
     // Sweep algorithm per direction: 0 = level-scheduled rows (k_sweep),
     // 1 = block-local over contiguous blocks of blk_rows rows (k_sweep_blk),
     // 2 = packed block-local over the current partition (k_sweep_pp, level
-    // barriers), 3 = the same with LDS value-flags, 4 = one workgroup walking
+    // barriers), 3 = the same with LDS value-flags (both as chunk streams,
+    // k_sweep_st, where every row has at most one entry per lane), 4 = one workgroup walking
     // the level schedule (k_sweep_lv; no partition), 5 = wave-specialised
     // block sweep over record streams (k_sweep_ws).
     int mode_l = 0, mode_u = 0;
     pilu::SweepPack pack_l, pack_u;
     pilu::SweepStream stream_l, stream_u;
     // Sweeps of a solver whose sweep shape was never set (sweep_default):
-    // level-scheduled rows at first, chunk streams after a few applies where
-    // the pattern suits them (auto_l / auto_u, decided for auto_pattern and
-    // the lanes).
+    // level-scheduled rows at first, chunk streams (auto_l / auto_u) or the level
+    // walk after a few applies where the pattern suits them (decided for
+    // auto_pattern and the lanes).
     bool sweep_default = true, auto_on = false, walk_on = false;
     int auto_applies = 0, auto_pattern = -1, auto_lanes[2] = {0, 0};
     pilu::SweepStream auto_l, auto_u;
