@@ -49,6 +49,7 @@
 
 #include "ilu_internal.hpp"
 #include "ilu_stream.hpp"
+#include "ilu_stream_plan.hpp"
 
 namespace pilu {
 
@@ -56,12 +57,7 @@ namespace {
 
 using Ext = lljbash::IluSolver::Ext;
 
-constexpr int kStSolvers = 8;     // solver waves per workgroup
-constexpr int kStThreads = 64 * (kStSolvers + 1);  // and one importer wave
-// Requests run kStAhead chunks (of the same wave) ahead for the slots, half
-// of that for the values, the diagonal and b, whose address comes with them.
-constexpr int kStAhead = 16;
-constexpr int kStAheadB = 8;
+constexpr int kStThreads = 64 * (kStSolvers + 1);  // solver waves and one importer wave
 constexpr size_t kStMaxLds = 160 * 1024;
 constexpr size_t kStMinLds = kStMaxLds / 2 + 1024;  // one workgroup per CU
 
@@ -124,8 +120,9 @@ struct StB {
 };
 
 // Raw buffer access: scalar base, one 32-bit byte offset per lane and a
-// scalar offset, so a chunk's requests need no address arithmetic; offsets
-// past `bytes` read 0 and store nothing.
+// scalar offset, so a chunk's requests need no address arithmetic.  A lane
+// offset past `bytes` (kStNone) reads 0 and stores nothing; scalar offsets stay
+// inside the buffer (kStOverrun).
 using Rsrc = __amdgpu_buffer_rsrc_t;
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -178,7 +175,7 @@ template <int G, typename T, bool UPPER>
 __global__ __launch_bounds__(kStThreads) void k_sweep_st(int n, const int* __restrict__ kptr,
                                                          const int* __restrict__ cptr,
                                                          const int2* __restrict__ irange, uint64_t* mail,
-                                                         unsigned mail_words, int* gen, unsigned nchunk,
+                                                         unsigned mail_words, int* gen, unsigned held,
                                                          const uint2* __restrict__ scol, const T* __restrict__ sval,
                                                          const double2* __restrict__ sdiag, const double* b,
                                                          double* out, const int* gate, int* ctr, int* err,
@@ -228,14 +225,14 @@ __global__ __launch_bounds__(kStThreads) void k_sweep_st(int n, const int* __res
         const uint64_t first_lanes = __ballot(first);
         const unsigned lds0 =
             static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) double*)xs));
-        const Rsrc r_col = st_rsrc(scol, nchunk * 512u);
-        const Rsrc r_val = st_rsrc(sval, nchunk * static_cast<unsigned>(64 * sizeof(T)));
-        const Rsrc r_diag = st_rsrc(sdiag, UPPER ? nchunk * static_cast<unsigned>(16 * R) : 0u);
+        const Rsrc r_col = st_rsrc(scol, held * 512u);
+        const Rsrc r_val = st_rsrc(sval, held * static_cast<unsigned>(64 * sizeof(T)));
+        const Rsrc r_diag = st_rsrc(sdiag, UPPER ? held * static_cast<unsigned>(16 * R) : 0u);
         const Rsrc r_b = st_rsrc(b, 8u * n), r_out = st_rsrc(out, 8u * n);
         const Rsrc r_box = st_rsrc(box, 8u * mail_words);
         const unsigned o_col = 8u * lane, o_val = sizeof(T) * lane, o_diag = 16u * (lane / G);
         // past a block's end the requests run into the next block's chunks
-        // (or the buffer's end), whose values are not used
+        // or the unused ones behind the last, whose values are not used
         unsigned ca = c0 + wave, cb = c0 + wave;  // next chunk of each kind to request
         auto issue_a = [&](StA& a) {
             a.p = st_load2(r_col, o_col, ca * 512u);
@@ -443,9 +440,10 @@ __global__ __launch_bounds__(256) void k_st_cut(int R, const int* __restrict__ b
 }
 
 // Stream of one lane: its x address and the factor entry it holds (-1:
-// none), and the row ids.  A chunk's block is found by bisection of cptr.
+// none), and the row ids.  A chunk's block is found by bisection of cptr;
+// the chunks past the last one hold nothing.
 template <bool UPPER>
-__global__ void k_st_fill(long nlanes, int G, int nblk, const int2* __restrict__ chunks, const int* __restrict__ cptr,
+__global__ void k_st_fill(long nlanes, int nchunk, int G, int nblk, const int2* __restrict__ chunks, const int* __restrict__ cptr,
                           const int* __restrict__ kptr, const int2* __restrict__ irange,
                           const int* __restrict__ escan, const int* __restrict__ refs,
                           const int* __restrict__ perm, const int* __restrict__ kinv, const int* __restrict__ rp,
@@ -456,6 +454,12 @@ __global__ void k_st_fill(long nlanes, int G, int nblk, const int2* __restrict__
     if (i >= nlanes) return;
     const int R = 64 / G;
     const int c = static_cast<int>(i >> 6), l = static_cast<int>(i & 63), j = l / G, t = l % G;
+    if (c >= nchunk) {
+        scol[i] = make_uint2(0, kStNone);
+        ssrc[i] = -1;
+        if (t == 0) srow[static_cast<long>(c) * R + j] = -1;
+        return;
+    }
     int lo = 0, hi = nblk;  // last block with cptr <= c
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
@@ -537,7 +541,7 @@ void launch_st(Ext* e, const SweepStream& st, const T* sval, const double* b, do
                                  static_cast<int>(st.lds)));
     kern<<<st.nblk, kStThreads, st.lds, e->stream>>>(
         e->n, st.kptr.get(), st.cptr.get(), reinterpret_cast<const int2*>(st.irange.get()), st.mail.get(),
-        static_cast<unsigned>(st.mail_words), st.gen.get(), static_cast<unsigned>(st.nchunk),
+        static_cast<unsigned>(st.mail_words), st.gen.get(), static_cast<unsigned>(st.nchunk + kStOverrun),
         reinterpret_cast<const uint2*>(st.scol.get()), sval, reinterpret_cast<const double2*>(st.sdiag.get()), b, out,
         gate, ctr, err, watchdog_ticks(e->watchdog_s));
 }
@@ -618,23 +622,22 @@ bool build_stream(Ext* e, bool upper, int G, const StreamSchedule& sc, SweepStre
     st.nchunk = h[nb1 + nblk];
     // every buffer has 32-bit byte offsets and the block fits the LDS (so
     // its slots 15 bits); the packed factors take the partition otherwise
-    if (lds > kStMaxLds || st.nchunk > (1L << 31) / 512 || st.mail_words >= (1L << 28) || n >= (1 << 28))
+    if (lds > kStMaxLds || st.nchunk + kStOverrun > (1L << 31) / 512 || st.mail_words >= (1L << 28) || n >= (1 << 28))
         return false;
     PILU_HIP(hipMemcpyAsync(st.irange.get(), h.data() + 2 * nb1, 2 * sizeof(int) * nblk, hipMemcpyHostToDevice, s));
-    const long nlanes = st.nchunk * 64;
+    const long held = st.nchunk + kStOverrun, nlanes = held * 64;
     int* rowlane = cnt.get();  // the counts have been scanned
     DevBuf<int> chunks(2 * static_cast<size_t>(std::max<long>(st.nchunk, 1)));
-    st.scol.reserve(2 * std::max<long>(nlanes, 1));
-    st.ssrc.reserve(std::max<long>(nlanes, 1));
-    st.srow.reserve(static_cast<size_t>(std::max<long>(st.nchunk * R, 1)));
+    st.scol.reserve(2 * nlanes);
+    st.ssrc.reserve(nlanes);
+    st.srow.reserve(held * R);
     k_st_cut<<<nblk, 256, 0, s>>>(R, blev, loff, st.cptr.get(), reinterpret_cast<int2*>(chunks.get()));
     auto fill = upper ? k_st_fill<true> : k_st_fill<false>;
-    if (nlanes > 0)
-        fill<<<grid_for(nlanes, 256), 256, 0, s>>>(
-            nlanes, G, nblk, reinterpret_cast<const int2*>(chunks.get()), st.cptr.get(), st.kptr.get(),
-            reinterpret_cast<const int2*>(irefs.get()), escan.get(), refs.get(), perm, kinv.get(), e->rp.get(),
-            e->dg.get(), e->ci.get(), block_of, reinterpret_cast<uint2*>(st.scol.get()), st.ssrc.get(),
-            st.srow.get(), rowlane);
+    fill<<<grid_for(nlanes, 256), 256, 0, s>>>(
+        nlanes, static_cast<int>(st.nchunk), G, nblk, reinterpret_cast<const int2*>(chunks.get()), st.cptr.get(),
+        st.kptr.get(), reinterpret_cast<const int2*>(irefs.get()), escan.get(), refs.get(), perm, kinv.get(),
+        e->rp.get(), e->dg.get(), e->ci.get(), block_of, reinterpret_cast<uint2*>(st.scol.get()), st.ssrc.get(),
+        st.srow.get(), rowlane);
     // every import becomes a mailbox word its row's lanes store to
     DevBuf<int> exported(static_cast<size_t>(n) + 1);
     PILU_HIP(hipMemsetAsync(exported.get(), 0, sizeof(int) * (static_cast<size_t>(n) + 1), s));
@@ -655,16 +658,16 @@ bool build_stream(Ext* e, bool upper, int G, const StreamSchedule& sc, SweepStre
 
 void gather_stream(Ext* e, bool upper, SweepStream& st) {
     refuse_if_no_alloc(e, "sweep stream values");
-    const long nlanes = st.nchunk * 64, nrow = st.nchunk * (64 / st.g);
-    if (upper) st.sdiag.reserve(2 * static_cast<size_t>(std::max<long>(nrow, 1)));
+    const long held = st.nchunk + kStOverrun, nlanes = held * 64, nrow = held * (64 / st.g);
+    if (upper) st.sdiag.reserve(2 * nrow);
     double2* sdiag = upper ? reinterpret_cast<double2*>(st.sdiag.get()) : nullptr;
     const int grid = 2048;
     if (e->precision == 32) {
-        st.sval32.reserve(std::max<long>(nlanes, 1));
+        st.sval32.reserve(nlanes);
         k_st_gather<float><<<grid, 256, 0, e->stream>>>(nlanes, st.ssrc.get(), e->fac32.get(), st.sval32.get(), nrow,
                                                         st.srow.get(), e->dg.get(), sdiag);
     } else {
-        st.sval64.reserve(std::max<long>(nlanes, 1));
+        st.sval64.reserve(nlanes);
         k_st_gather<double><<<grid, 256, 0, e->stream>>>(nlanes, st.ssrc.get(), e->fac.get(), st.sval64.get(), nrow,
                                                          st.srow.get(), e->dg.get(), sdiag);
     }
