@@ -554,11 +554,21 @@ public:
     // also keeps what the backward pass reads.
     void forward(int n, const int* rp, const int* ci, const double* va, float* omega, bool train = false) {
         prepare(n, rp, ci, va, train);
+        // k_layer reads an entry for rows that have none (and leaves it out): where
+        // there is no entry at all, the caller's columns may be null
+        const int* cols = ci;
+        if (nnz_ == 0) {
+            if (no_cols_.size() == 0) {
+                no_cols_.resize(1);
+                PILU_HIP(hipMemset(no_cols_.get(), 0, sizeof(int)));
+            }
+            cols = no_cols_.get();
+        }
         // a multiple of the 8 XCDs, at most 8 workgroups per CU
         const int grid = std::min((ceil_div(n, 64) + 7) / 8 * 8, 2048);
         auto run = [&](auto kern, int l) {
             const float* hin = l == 0 ? feat_.get() : h_[l - 1].get();
-            kern<<<grid, 256>>>(n, rp, ci, ew_.get(), hin, wb_.get() + gnn::kOffW[l], params_.get() + gnn::kOffB[l],
+            kern<<<grid, 256>>>(n, rp, cols, ew_.get(), hin, wb_.get() + gnn::kOffW[l], params_.get() + gnn::kOffB[l],
                                 h_[l].get(), m_[l].get(), params_.get(), omega);
         };
         if (train) {
@@ -665,6 +675,7 @@ private:
     long nnz_ = 0;
     DevBuf<unsigned short> wb_;
     DevBuf<double> dg_;
+    DevBuf<int> no_cols_;
     long step_ = 0;
 };
 

@@ -182,3 +182,21 @@ def test_uneven_rows_match_oracle(n):
     lref, gref = G.loss_grad(p.astype(np.float64), rp, ci, feat, w, t.astype(np.float64), True)
     assert loss == pytest.approx(lref, rel=2e-2)
     assert np.linalg.norm(g - gref) <= 3e-2 * np.linalg.norm(gref)
+
+
+@pytest.mark.parametrize("n", [1, 17, 130])
+def test_forward_without_entries(n):
+    """A graph without a single entry (its columns and values a null pointer):
+    every row has the features of an isolated node, so the oracle's value."""
+    import torch
+
+    p = np.random.default_rng(n).normal(0, 0.25, G.N_PARAMS).astype(np.float32)
+    net = Gnn(p)
+    none = np.zeros(0, np.int32)
+    rp = np.zeros(n + 1, np.int32)
+    (d_rp,) = dev(rp)
+    om = torch.zeros(n, dtype=torch.float32, device="cuda")
+    net.predict(n, d_rp.data_ptr(), 0, 0, om.data_ptr())
+    feat, w = G.features(rp, none, np.zeros(0))
+    ref, _, _ = G.forward(p.astype(np.float64), rp, none, feat, w, use_bf16=True)
+    assert np.max(np.abs(om.cpu().numpy() - ref)) <= 5e-3
