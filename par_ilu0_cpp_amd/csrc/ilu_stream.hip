@@ -58,8 +58,7 @@ namespace {
 using Ext = lljbash::IluSolver::Ext;
 
 constexpr int kStThreads = 64 * (kStSolvers + 1);  // solver waves and one importer wave
-constexpr size_t kStMaxLds = 160 * 1024;
-constexpr size_t kStMinLds = kStMaxLds / 2 + 1024;  // one workgroup per CU
+constexpr size_t kStMinLds = 81 * 1024;  // one workgroup per CU
 
 __device__ __forceinline__ void lds_put(double* xs, unsigned at, double v) {
     __hip_atomic_store(reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(xs) + at),
@@ -616,7 +615,7 @@ bool build_stream(Ext* e, bool upper, int G, const StreamSchedule& sc, SweepStre
         const size_t rows = h[p + 1] - h[p], imps = h[2 * nb1 + 2 * p + 1];
         h[2 * nb1 + 2 * p] = static_cast<int>(st.mail_words);
         st.mail_words += static_cast<long>(imps);
-        lds = std::max(lds, 8 * (rows + imps + 2));
+        lds = std::max(lds, st_block_lds(rows, imps));
         st.max_chunks = std::max(st.max_chunks, h[nb1 + p + 1] - h[nb1 + p]);
     }
     st.nchunk = h[nb1 + nblk];

@@ -2,6 +2,8 @@
 // plain C++ so that it can be checked on the host.
 #pragma once
 
+#include <cstddef>
+
 namespace pilu {
 
 constexpr int kStSolvers = 8;  // solver waves per workgroup; a block's chunks are a multiple of them
@@ -18,5 +20,12 @@ constexpr int kStAheadB = 8;
 // the scalar offset of a buffer request, which no range check is documented
 // to cover.
 constexpr long kStOverrun = kStSolvers * (2L * kStAhead - 1);
+
+// LDS of a block: a word per row and per import, and two for unused lanes and
+// rows.  The 160 KiB of a CU also hold the workgroup's ticket, a static word
+// that the dynamic part is aligned after.
+constexpr size_t kStStaticLds = 16;
+constexpr size_t kStMaxLds = 160 * 1024 - kStStaticLds;
+constexpr size_t st_block_lds(size_t rows, size_t imports) { return 8 * (rows + imports + 2); }
 
 }  // namespace pilu

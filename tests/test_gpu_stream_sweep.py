@@ -111,6 +111,30 @@ def test_row_imported_by_many_blocks(blocks, stream):
     assert ("lds_bytes" in ilu.Schedule()["pack_l"]) is stream
 
 
+@pytest.mark.parametrize("slots", [20477, 20478, 20479, 20480, 20481])
+def test_block_at_the_lds_limit(slots):
+    """A block of 16384 rows whose imports take its slots past the LDS of a CU:
+    chunk stream or packed factors, the level sweep's bits."""
+    blk, k = 16384, slots - 16384 - 2
+    n = blk + k
+    first = np.arange(n) < k
+    later = np.arange(n) >= blk
+    i = np.arange(n)
+    rp = np.concatenate([[0], np.cumsum(1 + first + later)]).astype(np.int32)
+    ci = np.concatenate([[r] if not (a or b) else [r, r + blk] if a else [r - blk, r]
+                         for r, a, b in zip(i, first, later)]).astype(np.int32)
+    va = np.where(ci == np.repeat(i, np.diff(rp)), 4.0, -0.5)
+    ilu = factored(rp, ci, va)
+    ilu.SetSweepLanes(4, 4)
+    b = np.random.default_rng(8).uniform(-1, 1, n)
+    want = ilu.Substitute(b)
+    ilu.SetSweepMode(2, 2, blk)
+    for _ in range(2):
+        assert np.array_equal(ilu.Substitute(b), want)
+    # U: block 0 imports the k rows of block 1
+    assert ("lds_bytes" in ilu.Schedule()["pack_u"]) == (slots <= 20478)
+
+
 def grid_matrix(nx, ny, nz, lof, oracle):
     """7-point (5-point for one plane) operator with its ILU(lof) pattern."""
     rng = np.random.default_rng(nx + 10 * ny + 100 * nz)

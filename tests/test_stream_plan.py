@@ -46,3 +46,15 @@ def test_requests_of_the_last_block_stay_in_the_buffers(tmp_path):
         }
     std::printf("%ld %ld %ld", worst_a, worst_b, kStOverrun);""")
     assert worst[0] == worst[2] and 0 < worst[1] < worst[2]
+
+
+def test_a_block_leaves_room_for_the_ticket(tmp_path):
+    """Slots (rows, imports and the two spare ones) of the largest block that
+    goes to a stream: with the kernel's static word a CU's 160 KiB hold 20479
+    at most, and 20480 must not be tried."""
+    fits = run(tmp_path, """
+    for (size_t slots = 20470; slots <= 20490; ++slots)
+        std::printf("%d ", st_block_lds(16384, slots - 16384 - 2) <= kStMaxLds);""")
+    most = 20470 + sum(fits) - 1
+    assert fits == sorted(fits, reverse=True) and 20478 <= most <= 20479
+    assert most * 8 + 4 <= 160 * 1024
