@@ -152,7 +152,8 @@ public:
     int CopyFillLevels(signed char* out) const;
     // The schedules and sweep configuration as one JSON object: levels per
     // direction, block rows and blocks, sweep mode and lanes per direction,
-    // packed entries (with padding) and passes.  Printed to stdout after
+    // packed entries (with padding) and passes, and the form a solver whose
+    // sweep shape was never set has taken ("default_sweeps").  Printed to stdout after
     // SetupMatrix and after a sweep-shape change when the environment
     // variable PAR_ILU_SHOW_ALGORITHM is set (the reference prints its
     // schedule under the SHOW_ALGORITHM macro, src/ilu_solver.cpp:196-223).

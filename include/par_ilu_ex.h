@@ -128,7 +128,16 @@ int IluSolverSymbolicDeviceEx(IluSolverHdl hdl, const CsrMatrix* d_a, int lof);
 #define IluSolverFactorizeDeviceEx LLJBASH_DECL(IluSolverFactorizeDeviceEx)
 int IluSolverFactorizeDeviceEx(IluSolverHdl hdl, const double* d_values, int values_are_a);
 
-/* x = U^-1 L^-1 b on device vectors (b may alias x). */
+/* x = U^-1 L^-1 b on device vectors (b may alias x).  Asynchronous, except
+ * where it has sweep structures to build: once after a change of sweep shape,
+ * and on a solver whose sweep shape was never set in its third apply of a
+ * pattern, in a GMRES solve or alone.  That one replaces the level-scheduled
+ * sweeps by faster ones where the pattern suits them: it allocates device
+ * memory (mostly one to three times the factors'), waits for the stream and
+ * takes as long as one to three applies before.  Results keep their bits.
+ * "default_sweeps" of IluSolverScheduleJsonEx tells the form in use ("level
+ * rows", "one workgroup", "tiles", "level walk") and its bytes;
+ * IluSolverSetSweepModeEx(hdl, 0, 0, 0) keeps the level-scheduled sweeps. */
 #define IluSolverSubstituteDeviceEx LLJBASH_DECL(IluSolverSubstituteDeviceEx)
 int IluSolverSubstituteDeviceEx(IluSolverHdl hdl, const double* d_b, double* d_x);
 

@@ -74,6 +74,10 @@ struct SweepStream {
     size_t lds = 0;
     int version = -1, g = 0;        // partition (default streams: pattern) and lanes per row it was built for
     long factors = -1;              // factorization its values were gathered from
+    size_t bytes() const {
+        return kptr.bytes() + cptr.bytes() + irange.bytes() + mail.bytes() + gen.bytes() + scol.bytes() + ssrc.bytes() +
+               srow.bytes() + sval64.bytes() + sdiag.bytes() + sval32.bytes();
+    }
 };
 
 // Streams of one direction's level walk (ilu_walk.hip), in the waves' step order.
@@ -89,6 +93,10 @@ struct WalkStream {
     int g = 0, p = 0, nlev = 0, ntask = 0, per = 0;  // p: entries per lane and step; per: tasks per wave
     int version = -1;                // pattern it was built for
     long factors = -1;               // factorization its values were gathered from
+    size_t bytes() const {
+        return perm.bytes() + toff.bytes() + first.bytes() + sbase.bytes() + ctl.bytes() + row.bytes() + brow.bytes() +
+               ref.bytes() + val64.bytes() + diag.bytes() + bt.bytes() + val32.bytes();
+    }
 };
 
 // Record streams of the wave-specialised sweep (mode 5) for one direction,

@@ -2736,7 +2736,16 @@ std::string IluSolver::DescribeSchedule() const {
                       static_cast<size_t>(160 * 1024) / std::max<size_t>(lds, 1));
         return std::string(b);
     };
-    js += ", \"ws_l\": " + ws(e->ws_l) + ", \"ws_u\": " + ws(e->ws_u) + "}";
+    js += ", \"ws_l\": " + ws(e->ws_l) + ", \"ws_u\": " + ws(e->ws_u);
+    // what a solver whose sweep shape was never set sweeps over now, and the
+    // memory that takes beside the factors
+    std::string form = "null";
+    if (e->sweep_default) {
+        const char* kind = e->auto_on ? (e->auto_l.nblk == 1 ? "one workgroup" : "tiles") : e->walk_on ? "level walk" : "level rows";
+        const size_t bytes = e->auto_l.bytes() + e->auto_u.bytes() + e->walk_l.bytes() + e->walk_u.bytes();
+        form = std::string("{\"form\": \"") + kind + "\", \"bytes\": " + std::to_string(bytes) + "}";
+    }
+    js += ", \"default_sweeps\": " + form + "}";
     return js;
 }
 

@@ -197,6 +197,33 @@ def test_default_sweeps_without_a_grid():
             assert np.array_equal(ilu.Substitute(b), first)
 
 
+@pytest.mark.parametrize("shape,form", [((40, 30, 1), "one workgroup"), ((150, 131, 1), "tiles"), (None, "level walk"),
+                                        ((7000, 1, 1), "level rows")])
+def test_schedule_reports_the_default_sweeps(oracle, shape, form):
+    """Level rows for two applies, then the form the pattern suits, and nothing
+    once a shape is set; the memory it holds is reported with it."""
+    if shape is None:
+        rp, ci, va = walk_pattern("rows", True)
+    elif form == "level rows":  # one entry per row: two levels of 3500 rows, nothing to gain
+        n = shape[0]
+        rows = [[i] if i < n // 2 else [i - n // 2, i] for i in range(n)]
+        rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+        ci = np.concatenate(rows).astype(np.int32)
+        va = np.where(ci == np.repeat(np.arange(n), np.diff(rp)), 2.0, -1.0)
+    else:
+        rp, ci, va = grid_matrix(*shape, 0, oracle)
+    ilu = factored(rp, ci, va)
+    b = np.random.default_rng(9).uniform(-1, 1, rp.size - 1)
+    first = ilu.Substitute(b)
+    for _ in range(2):
+        assert ilu.Schedule()["default_sweeps"]["form"] == "level rows"
+        assert np.array_equal(ilu.Substitute(b), first)
+    now = ilu.Schedule()["default_sweeps"]
+    assert now["form"] == form and (form == "level rows" or now["bytes"] > 0)
+    ilu.SetSweepMode(0, 0, 0)
+    assert ilu.Schedule()["default_sweeps"] is None
+
+
 def walk_pattern(kind, dominant):
     rng = np.random.default_rng(11)
     if kind == "chain":  # one row a level, dependencies both sides of the LDS ring's 16384 rows
