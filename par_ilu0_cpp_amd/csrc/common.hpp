@@ -16,6 +16,12 @@ namespace pilu {
 // ---------------------------------------------------------------------
 [[noreturn]] void hip_fail(hipError_t e, const char* what, const char* file, int line);
 
+// Device memory has run out: the one HIP failure that is answered by doing
+// without a structure where there is another way.
+struct OutOfDeviceMemory : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+
 #define PILU_HIP(call)                                                   \
     do {                                                                 \
         hipError_t pilu_e_ = (call);                                     \
@@ -30,6 +36,11 @@ namespace pilu {
 // scope must be ordered on that one stream.
 void* dev_alloc(size_t bytes);
 void dev_free(void* p, size_t bytes);
+
+// The calling thread's dev_alloc call after the next `calls` ones fails as if
+// device memory had run out; a negative number stops that.  For tests: no
+// other code calls it.
+extern "C" void par_ilu_fail_allocation(long calls);
 
 class SetupScope {
 public:

@@ -36,6 +36,10 @@ namespace pilu {
     char buf[512];
     std::snprintf(buf, sizeof(buf), "HIP error %d (%s) in %s at %s:%d", static_cast<int>(e),
                   hipGetErrorString(e), what, file, line);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();  // the exception carries it: no later check should find it
+        throw OutOfDeviceMemory(buf);
+    }
     throw std::runtime_error(buf);
 }
 
@@ -150,9 +154,14 @@ BlockPool& pool() {
     static BlockPool* p = new BlockPool;
     return *p;
 }
+
+thread_local long g_fail_in = -1;  // dev_alloc calls until one fails (par_ilu_fail_allocation)
 }  // namespace
 
+extern "C" void par_ilu_fail_allocation(long calls) { g_fail_in = calls; }
+
 void* dev_alloc(size_t bytes) {
+    if (g_fail_in >= 0 && g_fail_in-- == 0) hip_fail(hipErrorOutOfMemory, "dev_alloc", __FILE__, __LINE__);
     if (g_scope.depth > 0) {
         size_t best = 0;
         int at = -1;
@@ -263,6 +272,11 @@ void refuse_if_no_alloc(const lljbash::IluSolver::Ext* e, const char* what) {
 }
 
 namespace {
+
+// The rows cannot be partitioned as asked, or not in time.
+struct NoPartition : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
 
 // f(begin, end) over [0, n) in contiguous chunks on up to 16 host threads.
 template <typename F>
@@ -432,11 +446,11 @@ void build_block_schedule(Ext* e, bool upper, const int* block_of, int nblk, con
     PILU_HIP(hipGetLastError());
     const int nlev = read_int(maxlev, s) + 1;
     if (read_int(e->err.get() + kErrLevels, s) & kErrTimeout)
-        throw std::runtime_error("block level analysis: dependency wait timed out (watchdog)");
+        throw NoPartition("block level analysis: dependency wait timed out (watchdog)");
     int lbits = 1, pbits = 1;
     while ((1 << lbits) < nlev) ++lbits;
     while ((1 << pbits) < nblk) ++pbits;
-    if (lbits + pbits > 31) throw std::runtime_error("block schedule: too many blocks x levels");
+    if (lbits + pbits > 31) throw NoPartition("block schedule: too many blocks x levels");
     DevBuf<int> dpos(nblk);
     PILU_HIP(hipMemcpy(dpos.get(), pos.data(), sizeof(int) * nblk, hipMemcpyHostToDevice));
     DevBuf<unsigned> keys(n), keys_out(n);
@@ -596,7 +610,7 @@ std::vector<int> block_order(Ext* e, bool upper) {
         }
     }
     if (static_cast<int>(queue.size()) != nblk)
-        throw std::runtime_error("sweep partition: the block dependency graph has a cycle");
+        throw NoPartition("sweep partition: the block dependency graph has a cycle");
     std::vector<int> order(nblk);
     for (int b = 0; b < nblk; ++b) order[b] = b;
     std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return depth[a] < depth[c]; });
@@ -648,7 +662,7 @@ void install_partition(Ext* e, int nblk, bool contiguous) {
         e->max_block_rows = *std::max_element(hc.begin(), hc.end());
     }
     if (e->max_block_rows > kMaxBlockRows)
-        throw std::runtime_error("sweep partition: a block holds more than 16384 rows");
+        throw NoPartition("sweep partition: a block holds more than 16384 rows");
     std::vector<int> pos_l(nblk), pos_u(nblk);
     if (contiguous) {
         for (int b = 0; b < nblk; ++b) {
@@ -792,7 +806,7 @@ void use_tiles(Ext* e, int tx, int ty, int tz) {
     pt.mark("skew");
     const long umax = (nx - 1) + b * (ny - 1) + c * (nz - 1), vmax = (ny - 1) + c2 * (nz - 1);
     const long ntu = umax / tx + 1, ntv = vmax / ty + 1, ntw = (nz - 1) / tz + 1;
-    if (ntu * ntv * ntw > (1L << 30)) throw std::runtime_error("tiled sweeps: too many tiles");
+    if (ntu * ntv * ntw > (1L << 30)) throw NoPartition("tiled sweeps: too many tiles");
     const int ntiles = static_cast<int>(ntu * ntv * ntw);
     // tile of every row and the first row of every tile on the device; the
     // non-empty tiles get dense ids in order of their first row
@@ -1891,34 +1905,8 @@ bool build_auto_walk(Ext* e, int gl, int gu) {
     return build_walk(e, false, gl, e->walk_l) && build_walk(e, true, gu, e->walk_u);
 }
 
-bool build_auto_stream(Ext* e, int gl, int gu) {
-    if (!stream_width_fits(e, false, gl) || !stream_width_fits(e, true, gu)) return false;
-    const int n = e->n;
-    hipStream_t s = e->stream;
-    const long level_rows = static_cast<long>(64 / std::max(gl, gu)) * std::min(e->nlev_l, e->nlev_u);
-    auto one_block = [&]() {
-        DevBuf<int> block_of(n), blev(4);
-        const int hb[4] = {0, e->nlev_l, 0, e->nlev_u};
-        PILU_HIP(hipMemcpyAsync(blev.get(), hb, sizeof(hb), hipMemcpyHostToDevice, s));
-        k_fill_int<<<grid_for(n, 256 * 8), 256, 0, s>>>(n, block_of.get(), 0);
-        return build_stream(e, false, gl, {e->perm_l.get(), blev.get(), e->lvoff_l.get(), block_of.get(), 1}, e->auto_l) &&
-               build_stream(e, true, gu, {e->perm_u.get(), blev.get() + 2, e->lvoff_u.get(), block_of.get(), 1}, e->auto_u);
-    };
-    if (n <= kMaxBlockRows && n <= kAutoNarrow * level_rows) return one_block();
-    DevBuf<int> tab(kOffsets + 1);
-    k_fill_int<<<1, 64, 0, s>>>(kOffsets + 1, tab.get(), 0);
-    k_offsets<<<std::min(grid_for(n, 256), kOffsetBlocks), 256, 0, s>>>(n, e->rp.get(), e->dg.get(), e->ci.get(), tab.get(), tab.get() + kOffsets);
-    PILU_HIP(hipGetLastError());
-    int h[kOffsets + 1];
-    PILU_HIP(hipMemcpyAsync(h, tab.get(), sizeof(h), hipMemcpyDeviceToHost, s));
-    PILU_HIP(hipStreamSynchronize(s));
-    std::vector<int> d;
-    for (int k = 0; k < kOffsets; ++k)
-        if (h[k] != 0) d.push_back(h[k]);
-    std::sort(d.begin(), d.end());
-    int shape[3];
-    if (h[kOffsets] || !infer_grid(n, d, shape))
-        return n <= kMaxBlockRows && n <= kAutoWide * level_rows && one_block();
+// Chunk streams over tiles of the natural-order grid `shape`.
+bool build_grid_stream(Ext* e, int gl, int gu, const int* shape) {
     // the partition is only needed for the build: what describes a configured
     // one is put back
     struct Restore {
@@ -1951,27 +1939,95 @@ bool build_auto_stream(Ext* e, int gl, int gu) {
            build_stream(e, true, gu, {e->bperm_u.get(), e->blev_u.get(), e->loff_u.get(), e->block_of.get(), e->nblk}, e->auto_u);
 }
 
+bool build_auto_stream(Ext* e, int gl, int gu) {
+    if (!stream_width_fits(e, false, gl) || !stream_width_fits(e, true, gu)) return false;
+    const int n = e->n;
+    hipStream_t s = e->stream;
+    const long level_rows = static_cast<long>(64 / std::max(gl, gu)) * std::min(e->nlev_l, e->nlev_u);
+    auto one_block = [&]() {
+        DevBuf<int> block_of(n), blev(4);
+        const int hb[4] = {0, e->nlev_l, 0, e->nlev_u};
+        PILU_HIP(hipMemcpyAsync(blev.get(), hb, sizeof(hb), hipMemcpyHostToDevice, s));
+        k_fill_int<<<grid_for(n, 256 * 8), 256, 0, s>>>(n, block_of.get(), 0);
+        return build_stream(e, false, gl, {e->perm_l.get(), blev.get(), e->lvoff_l.get(), block_of.get(), 1}, e->auto_l) &&
+               build_stream(e, true, gu, {e->perm_u.get(), blev.get() + 2, e->lvoff_u.get(), block_of.get(), 1}, e->auto_u);
+    };
+    if (n <= kMaxBlockRows && n <= kAutoNarrow * level_rows) return one_block();
+    DevBuf<int> tab(kOffsets + 1);
+    k_fill_int<<<1, 64, 0, s>>>(kOffsets + 1, tab.get(), 0);
+    k_offsets<<<std::min(grid_for(n, 256), kOffsetBlocks), 256, 0, s>>>(n, e->rp.get(), e->dg.get(), e->ci.get(), tab.get(), tab.get() + kOffsets);
+    PILU_HIP(hipGetLastError());
+    int h[kOffsets + 1];
+    PILU_HIP(hipMemcpyAsync(h, tab.get(), sizeof(h), hipMemcpyDeviceToHost, s));
+    PILU_HIP(hipStreamSynchronize(s));
+    std::vector<int> d;
+    for (int k = 0; k < kOffsets; ++k)
+        if (h[k] != 0) d.push_back(h[k]);
+    std::sort(d.begin(), d.end());
+    int shape[3];
+    if (!h[kOffsets] && infer_grid(n, d, shape)) {
+        try {
+            return build_grid_stream(e, gl, gu, shape);
+        } catch (const NoPartition&) {
+            // a pattern whose offsets only look like a grid's
+        }
+    }
+    return n <= kMaxBlockRows && n <= kAutoWide * level_rows && one_block();
+}
+
+void drop_auto(Ext* e) {
+    e->auto_on = e->walk_on = false;
+    for (SweepStream* st : {&e->auto_l, &e->auto_u}) *st = SweepStream{};
+    for (WalkStream* w : {&e->walk_l, &e->walk_u}) *w = WalkStream{};
+}
+
+// Values of the streams in use from the factors, for both directions at once,
+// so that an apply has them in both or in none; level-scheduled rows, which
+// need no more than the factors, take over where memory runs out.
+void refresh_auto(Ext* e) {
+    try {
+        for (const bool upper : {false, true}) {
+            SweepStream& st = upper ? e->auto_u : e->auto_l;
+            WalkStream& w = upper ? e->walk_u : e->walk_l;
+            if (e->auto_on && st.version == e->pattern_version && st.factors != e->factor_version) gather_stream(e, upper, st);
+            if (e->walk_on && w.version == e->pattern_version && w.factors != e->factor_version) gather_walk(e, upper, w);
+        }
+    } catch (const OutOfDeviceMemory&) {
+        drop_auto(e);
+    }
+}
+
 // Counts an apply of a default-shaped solver and decides once per pattern
-// and lane count.
+// and lane count.  The apply's own structures are there already, so where
+// memory runs out on the way nothing is lost: what was built is given back.
 void count_default_apply(Ext* e) {
     if (!e->sweep_default || e->mode_l != 0 || e->mode_u != 0) return;
     const int gl = effective_lanes(e, false), gu = effective_lanes(e, true);
     if (e->auto_pattern == e->pattern_version && e->auto_lanes[0] == gl && e->auto_lanes[1] == gu) return;
     if (e->auto_applies++ < kAutoAfter) return;
     SetupScope scope(e->stream);
-    e->auto_on = e->walk_on = false;
+    drop_auto(e);
     e->auto_pattern = e->pattern_version;
     e->auto_lanes[0] = gl;
     e->auto_lanes[1] = gu;
-    try {
-        e->auto_on = build_auto_stream(e, gl, gu);
-        if (!e->auto_on) e->walk_on = build_auto_walk(e, gl, gu);
-    } catch (const std::runtime_error&) {
-        // no acyclic tiles, or no memory for the streams: level-scheduled rows stay
-        (void)hipGetLastError();
-    }
-    e->auto_l.version = e->auto_u.version = e->auto_on ? e->pattern_version : -1;
-    e->walk_l.version = e->walk_u.version = e->walk_on ? e->pattern_version : -1;
+    auto attempt = [&](auto build, bool& on) {
+        try {
+            if (build(e, gl, gu)) {
+                on = true;
+                e->auto_l.version = e->auto_u.version = e->walk_l.version = e->walk_u.version = e->pattern_version;
+                refresh_auto(e);
+            } else {
+                drop_auto(e);
+            }
+        } catch (const OutOfDeviceMemory&) {
+            drop_auto(e);
+        } catch (...) {
+            drop_auto(e);
+            throw;
+        }
+        return on;
+    };
+    if (!attempt(build_auto_stream, e->auto_on)) attempt(build_auto_walk, e->walk_on);
 }
 
 // The stream that replaces the level-scheduled sweep of a direction, or null.
@@ -1980,8 +2036,8 @@ const SweepStream* auto_stream(Ext* e, bool upper) {
     if (!e->sweep_default || !e->auto_on || st.version != e->pattern_version ||
         st.g != effective_lanes(e, upper))
         return nullptr;
-    if (e->factored && st.factors != e->factor_version) gather_stream(e, upper, st);
-    return &st;
+    if (e->factored) refresh_auto(e);
+    return e->auto_on ? &st : nullptr;
 }
 
 // The same for the level walk.
@@ -1989,8 +2045,8 @@ const WalkStream* auto_walk(Ext* e, bool upper) {
     WalkStream& w = upper ? e->walk_u : e->walk_l;
     if (!e->sweep_default || !e->walk_on || w.version != e->pattern_version || w.g != effective_lanes(e, upper))
         return nullptr;
-    if (e->factored && w.factors != e->factor_version) gather_walk(e, upper, w);
-    return &w;
+    if (e->factored) refresh_auto(e);
+    return e->walk_on ? &w : nullptr;
 }
 
 template <typename T, bool UPPER>
@@ -2135,12 +2191,9 @@ bool run_factor(Ext* e) {
     gather_pack(e, e->pack_u, true);
     for (const bool upper : {false, true}) {
         SweepStream& st = upper ? e->stream_u : e->stream_l;
-        SweepStream& at = upper ? e->auto_u : e->auto_l;
         if (st.version == e->part_version && st.lds > 0) gather_stream(e, upper, st);
-        if (e->sweep_default && at.version == e->pattern_version && at.lds > 0) gather_stream(e, upper, at);
-        WalkStream& w = upper ? e->walk_u : e->walk_l;
-        if (e->sweep_default && e->walk_on && w.version == e->pattern_version) gather_walk(e, upper, w);
     }
+    if (e->sweep_default) refresh_auto(e);
     if (ws_current(e, e->ws_l, e->ws_l.g)) gather_ws(e, e->ws_l);
     if (ws_current(e, e->ws_u, e->ws_u.g)) gather_ws(e, e->ws_u);
     return (err & 1) == 0 && e->factor_status == 0;

@@ -282,3 +282,64 @@ def test_level_walk_keeps_the_bits_of_level_rows(kind, lanes, dominant, bits):
     again = ilu.Substitute(b)
     ilu.SetSweepMode(0, 0, 0)
     assert np.array_equal(ilu.Substitute(b), again, equal_nan=True)
+
+
+def fail_allocation(calls):
+    """The library's allocation after the next `calls` ones fails as if device memory had run out."""
+    import ctypes
+
+    from par_ilu0_cpp_amd import _lib
+
+    ctypes.CDLL(str(_lib.LIB_DIR / _lib.CORE_NAME)).par_ilu_fail_allocation(ctypes.c_long(calls))
+
+
+@pytest.mark.parametrize("kind", ["one workgroup", "tiles", "level walk"])
+def test_default_sweeps_without_memory(oracle, kind):
+    """Whichever allocation of the third apply fails, that apply and the next
+    ones have the level rows' result, and level rows hold nothing of what was
+    built; the same where the values of another precision find no memory."""
+    if kind == "level walk":
+        rp, ci, va = walk_pattern("few", True)
+    else:
+        rp, ci, va = grid_matrix(*((20, 15, 1) if kind == "one workgroup" else (30, 31, 16)), 0, oracle)
+    b = np.random.default_rng(10).uniform(-1, 1, rp.size - 1)
+
+    def default():
+        return ilu.Schedule()["default_sweeps"]
+
+    k = 0
+    while True:
+        ilu = factored(rp, ci, va)
+        first = ilu.Substitute(b)
+        ilu.Substitute(b)
+        fail_allocation(k)
+        try:
+            third = ilu.Substitute(b)
+        finally:
+            fail_allocation(-1)
+        assert np.array_equal(third, first), k
+        assert np.array_equal(ilu.Substitute(b), first), k
+        if default()["form"] == kind:
+            break
+        assert default()["form"] != "level rows" or default()["bytes"] == 0, k
+        k += 1
+        assert k < 300
+    assert k > 10
+    for k in range(8):
+        other = factored(rp, ci, va)
+        for _ in range(4):
+            other.Substitute(b)
+        assert other.Schedule()["default_sweeps"]["form"] == kind
+        other.SetFactorPrecision(32)
+        P.fill_csr(other.GetMatrix(), rp, ci, va)  # its values are the factors by now
+        fail_allocation(k)
+        try:
+            done = other.Factorize() == 0
+        finally:
+            fail_allocation(-1)
+        if not done:  # no memory for the factors themselves
+            P.fill_csr(other.GetMatrix(), rp, ci, va)
+            assert other.Factorize() == 0
+        want = factored(rp, ci, va, 32).Substitute(b)
+        for _ in range(3):
+            assert np.array_equal(other.Substitute(b), want), k
