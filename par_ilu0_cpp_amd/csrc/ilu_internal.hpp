@@ -4,6 +4,7 @@
 #include "common.hpp"
 #include "ilu_solver.hpp"
 
+#include <algorithm>
 #include <vector>
 
 namespace pilu {
@@ -208,4 +209,10 @@ struct lljbash::IluSolver::Ext {
     bool analysed = false;  // pattern checked and schedules built (SetupMatrix / SymbolicDevice completed)
     bool factored = false;
     bool y_armed = false;
+
+    // Bytes that a direction's stream (chunk stream or level walk) may take: a
+    // stream holds whole waves however few rows a level has, up to 2 KB per row
+    // where the factors of a chain have 36 bytes.  Grids take 1 to 3 times their
+    // factors, random bands about the same; 8 times, or 256 MiB for the small.
+    size_t stream_budget() const { return std::max(size_t{256} << 20, 8 * 12 * static_cast<size_t>(nnz)); }
 };

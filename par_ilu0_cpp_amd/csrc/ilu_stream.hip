@@ -623,8 +623,11 @@ bool build_stream(Ext* e, bool upper, int G, const StreamSchedule& sc, SweepStre
     // its slots 15 bits); the packed factors take the partition otherwise
     if (lds > kStMaxLds || st.nchunk + kStOverrun > (1L << 31) / 512 || st.mail_words >= (1L << 28) || n >= (1 << 28))
         return false;
-    PILU_HIP(hipMemcpyAsync(st.irange.get(), h.data() + 2 * nb1, 2 * sizeof(int) * nblk, hipMemcpyHostToDevice, s));
     const long held = st.nchunk + kStOverrun, nlanes = held * 64;
+    // slots, source, value; per row its id and the diagonal; two generations of mailboxes
+    const size_t lane_bytes = sizeof(uint2) + sizeof(int) + sizeof(double), row_bytes = sizeof(int) + 2 * sizeof(double);
+    if (nlanes * lane_bytes + held * R * row_bytes + 2 * sizeof(uint64_t) * st.mail_words > e->stream_budget()) return false;
+    PILU_HIP(hipMemcpyAsync(st.irange.get(), h.data() + 2 * nb1, 2 * sizeof(int) * nblk, hipMemcpyHostToDevice, s));
     int* rowlane = cnt.get();  // the counts have been scanned
     DevBuf<int> chunks(2 * static_cast<size_t>(std::max<long>(st.nchunk, 1)));
     st.scol.reserve(2 * nlanes);

@@ -18,7 +18,8 @@ bool stream_width_fits(const lljbash::IluSolver::Ext* e, bool upper, int G);
 
 // Builds the pattern part of a stream for G lanes per row
 // (stream_width_fits); false, with st.lds == 0, where a block does not fit
-// the LDS or a row is imported by more blocks than it has lanes for.
+// the LDS, a row is imported by more blocks than it has lanes for or the
+// stream exceeds its budget of memory.
 bool build_stream(lljbash::IluSolver::Ext* e, bool upper, int G, const StreamSchedule& sc, SweepStream& st);
 
 // Refreshes the values of a built stream from the factors.

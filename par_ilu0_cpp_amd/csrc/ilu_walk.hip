@@ -471,6 +471,9 @@ bool build_walk(Ext* e, bool upper, int G, WalkStream& w) {
     PILU_HIP(hipMemcpyAsync(&total, w.first.get() + nt - 1, sizeof(int), hipMemcpyDeviceToHost, s));
     PILU_HIP(hipStreamSynchronize(s));
     const size_t held = static_cast<size_t>(total) + 2 * kWalkAhead;
+    // slots and values of the entries; per row its id, twice, b and the diagonal
+    const size_t step_bytes = 64 * P * sums_of(G) * (sizeof(int) + sizeof(double)) + R * (2 * sizeof(int) + 3 * sizeof(double)) + sizeof(int2);
+    if (held * step_bytes > e->stream_budget()) return false;
     w.ctl.reserve(held);
     w.row.reserve(held * R);
     w.brow.reserve(held * R);

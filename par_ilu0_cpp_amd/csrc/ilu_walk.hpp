@@ -6,7 +6,8 @@
 namespace pilu {
 
 // Builds the pattern part of a direction's stream for G (>= 4) lanes per row;
-// false where a level is too wide for the LDS ring.
+// false where a level is too wide for the LDS ring or the stream exceeds its
+// budget of memory.
 bool build_walk(lljbash::IluSolver::Ext* e, bool upper, int G, WalkStream& w);
 
 // Refreshes the values of a built stream from the factors.

@@ -343,3 +343,41 @@ def test_default_sweeps_without_memory(oracle, kind):
         want = factored(rp, ci, va, 32).Substitute(b)
         for _ in range(3):
             assert np.array_equal(other.Substitute(b), want), k
+
+
+def tridiagonal(n):
+    i = np.arange(n)
+    cols = np.stack([i - 1, i, i + 1], 1)
+    keep = (cols >= 0) & (cols < n)
+    rp = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.int32)
+    return rp, cols[keep].astype(np.int32), np.broadcast_to([-1.0, 2.5, -1.0], (n, 3))[keep].copy()
+
+
+@pytest.mark.parametrize("n,form", [(130000, "level walk"), (131000, "level rows")])
+def test_level_walk_memory_is_bounded(n, form):
+    """A chain takes a whole wave's step per row: 2056 bytes of its stream per
+    row and direction, up to 256 MiB."""
+    rp, ci, va = tridiagonal(n)
+    ilu = factored(rp, ci, va)
+    b = np.random.default_rng(12).uniform(-1, 1, n)
+    first = ilu.Substitute(b)
+    for _ in range(3):
+        assert np.array_equal(ilu.Substitute(b), first)
+    now = ilu.Schedule()["default_sweeps"]
+    assert now["form"] == form
+    assert now["bytes"] < 2 * (256 << 20) + 24 * n if form == "level walk" else now["bytes"] == 0
+
+
+@pytest.mark.parametrize("n,stream", [(139000, True), (141000, False)])
+def test_chunk_stream_memory_is_bounded(n, stream):
+    """A chain takes a chunk per row: 64 lanes of 20 bytes and 32 row slots of
+    20; past 256 MiB the packed factors are swept."""
+    rp, ci, va = tridiagonal(n)
+    ilu = factored(rp, ci, va)
+    ilu.SetSweepLanes(2, 2)
+    b = np.random.default_rng(13).uniform(-1, 1, n)
+    ilu.SetSweepMode(2, 2, 4096)
+    got = ilu.Substitute(b)
+    assert ("lds_bytes" in ilu.Schedule()["pack_l"]) is stream
+    ilu.SetSweepMode(0, 0, 0)
+    assert np.array_equal(ilu.Substitute(b), got)
