@@ -774,8 +774,18 @@ __global__ void k_apply_tile_id(int n, const int* __restrict__ tile_of, const in
 // and the tiles form an acyclic graph.  A 7-point ILU(0) pattern gives
 // b = c = c2 = 0 (plain boxes); ILU(1), whose fill couples (x+1, y-1),
 // (x+1, z-1) and (y+1, z-1), gives b = c = c2 = 1.  The skew is unimodular,
-// so an interior tile holds exactly tx ty tz rows.
-void use_tiles(Ext* e, int tx, int ty, int tz) {
+// so an interior tile holds exactly tx ty tz rows.  Boxes without rows count
+// too: entries that wrap from one end of an axis to the other, and a short x
+// axis, stretch u far past the rows.  `guessed`: the grid was read off the
+// offsets of the entries; more boxes than rows and kGuessedTiles are refused
+// then.  A band of offsets 1 and 2, taken for a grid of nx = 2, has n^2 / 256
+// boxes: 14M at 60k rows, where the third apply spent 33 ms on them and tiles
+// then took 43 ms per apply (the level walk 31.5), 350M at 300k.  3M boxes (a
+// 40^3 stencil with entries that wrap) cost 5 ms and are worth it: 21.9 ms per
+// apply, 33.9 by the walk.
+constexpr long kGuessedTiles = 1L << 22;
+
+void use_tiles(Ext* e, int tx, int ty, int tz, bool guessed) {
     const int nx = e->grid[0], ny = e->grid[1], nz = e->grid[2];
     if (nx <= 0) throw std::runtime_error("tiled sweeps need the grid shape (SetGridShape)");
     if (tx < 1 || ty < 1 || tz < 1 || static_cast<long>(tx) * ty * tz > kMaxBlockRows)
@@ -807,6 +817,8 @@ void use_tiles(Ext* e, int tx, int ty, int tz) {
     const long umax = (nx - 1) + b * (ny - 1) + c * (nz - 1), vmax = (ny - 1) + c2 * (nz - 1);
     const long ntu = umax / tx + 1, ntv = vmax / ty + 1, ntw = (nz - 1) / tz + 1;
     if (ntu * ntv * ntw > (1L << 30)) throw NoPartition("tiled sweeps: too many tiles");
+    if (guessed && ntu * ntv * ntw > std::max<long>(n, kGuessedTiles))
+        throw NoPartition("tiled sweeps: many more tiles than rows");
     const int ntiles = static_cast<int>(ntu * ntv * ntw);
     // tile of every row and the first row of every tile on the device; the
     // non-empty tiles get dense ids in order of their first row
@@ -1933,8 +1945,8 @@ bool build_grid_stream(Ext* e, int gl, int gu, const int* shape) {
     // against 457 for 128 x 4 x 4) and the fastest at 77 x 59 x 91 (286, 305)
     // and at 128^3 ILU(0) (310, 349); 256 x 32 in 2D (512 x 400 ILU(1): 413 us,
     // 425 for 128 x 32)
-    if (shape[2] == 1) use_tiles(e, std::min(shape[0], 256), 32, 1);
-    else use_tiles(e, std::min(shape[0], 128), 8, 4);
+    if (shape[2] == 1) use_tiles(e, std::min(shape[0], 256), 32, 1, true);
+    else use_tiles(e, std::min(shape[0], 128), 8, 4, true);
     return build_stream(e, false, gl, {e->bperm_l.get(), e->blev_l.get(), e->loff_l.get(), e->block_of.get(), e->nblk}, e->auto_l) &&
            build_stream(e, true, gu, {e->bperm_u.get(), e->blev_u.get(), e->loff_u.get(), e->block_of.get(), e->nblk}, e->auto_u);
 }
@@ -2644,7 +2656,7 @@ int IluSolver::AutotuneSweeps(int reps, double* table, int cap) {
     for (size_t ip = 0; ip < parts.size(); ++ip) {
         const Part& pt = parts[ip];
         if (pt.blk) pilu::use_blocks(e, pt.blk);
-        else pilu::use_tiles(e, pt.tx, pt.ty, pt.tz);
+        else pilu::use_tiles(e, pt.tx, pt.ty, pt.tz, false);
         double bb[2] = {1e300, 1e300};
         int bl[2] = {8, 8}, bm[2] = {1, 1};
         if (pt.blk) {
@@ -2694,7 +2706,7 @@ int IluSolver::AutotuneSweeps(int reps, double* table, int cap) {
     if (pick >= 0) {
         const Part& pt = parts[pick];
         if (pt.blk) pilu::use_blocks(e, pt.blk);
-        else pilu::use_tiles(e, pt.tx, pt.ty, pt.tz);
+        else pilu::use_tiles(e, pt.tx, pt.ty, pt.tz, false);
     }
     e->mode_l = pick_mode[0];
     e->mode_u = pick_mode[1];
@@ -2734,7 +2746,7 @@ void IluSolver::SetSweepTiles(int mode_l, int mode_u, int tx, int ty, int tz) {
     auto ok = [](int m) { return m == 0 || m == 2 || m == 3 || m == 5; };
     if (!ok(mode_l) || !ok(mode_u)) throw std::runtime_error("tiled sweeps use mode 0, 2, 3 or 5");
     e->sweep_default = false;
-    pilu::use_tiles(e, tx, ty, tz);
+    pilu::use_tiles(e, tx, ty, tz, false);
     e->mode_l = mode_l;
     e->mode_u = mode_u;
     pilu::prepare_modes(e);

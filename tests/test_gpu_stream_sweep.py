@@ -381,3 +381,21 @@ def test_chunk_stream_memory_is_bounded(n, stream):
     assert ("lds_bytes" in ilu.Schedule()["pack_l"]) is stream
     ilu.SetSweepMode(0, 0, 0)
     assert np.array_equal(ilu.Substitute(b), got)
+
+
+@pytest.mark.parametrize("n,form", [(20000, "tiles"), (60000, "level walk")])
+def test_bands_taken_for_a_grid_have_few_tiles(n, form):
+    """Offsets 1 and 2 look like a grid two cells wide, whose skewed boxes grow
+    with the square of the rows: 1.6 million here, 14 million past the bound."""
+    i = np.arange(n)
+    cols = i[:, None] + np.arange(-2, 3)
+    keep = (cols >= 0) & (cols < n)
+    rp = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.int32)
+    ci = cols[keep].astype(np.int32)
+    va = np.broadcast_to([-0.5, -1.0, 4.0, -1.0, -0.5], (n, 5))[keep].copy()
+    ilu = factored(rp, ci, va)
+    b = np.random.default_rng(14).uniform(-1, 1, n)
+    first = ilu.Substitute(b)
+    for _ in range(3):
+        assert np.array_equal(ilu.Substitute(b), first)
+    assert ilu.Schedule()["default_sweeps"]["form"] == form
