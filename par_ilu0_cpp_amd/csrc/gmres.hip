@@ -838,7 +838,8 @@ std::pair<bool, int> solve_core(GExt* e, IluSolver* ilu, const std::function<voi
                         nullptr);
     pilu::k_sqrt_sum<<<1, pilu::kVecThreads, 0, s>>>(part0, np, part1);
     PILU_HIP(hipMemcpyAsync(&e->true_res, part1, sizeof(double), hipMemcpyDeviceToHost, s));
-    if (ie) pilu::check_sweep_errors(ie);
+    if (ie) pilu::check_sweep_errors(ie);  // waits for the stream
+    else PILU_HIP(hipStreamSynchronize(s));
     if (mgs.nwg > 0) {  // cooperative launches may have run (before a refusal too)
         int werr = 0;
         PILU_HIP(hipMemcpyAsync(&werr, mgs_err, sizeof(int), hipMemcpyDeviceToHost, s));

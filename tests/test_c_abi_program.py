@@ -135,3 +135,33 @@ def test_cpp_reference_layout_precon_paths_agree(tmp_path):
     # the host-callback path applies the same sweeps to the same vectors
     assert its[0] == its[1] == its[2] and its[0] > 0, its
     assert float(f["max_diff"][0]) == 0.0
+
+
+HOST_PRECON = ROOT / "tests" / "c_abi" / "host_precon.cpp"
+
+
+def build_host_precon(out: Path) -> Path:
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no C++ compiler")
+    exe = out / "host_precon"
+    cmd = [cxx, "-std=c++17", "-Wall", "-Werror", "-O2", f"-I{ROOT / 'include'}", str(HOST_PRECON), "-o", str(exe),
+           f"-L{LIB}", "-lpar-ilu0-gmres", f"-Wl,-rpath,{LIB}"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    return exe
+
+
+def test_cpp_host_precon_program_compiles(tmp_path):
+    build_host_precon(tmp_path)
+
+
+@pytest.mark.gpu
+def test_cpp_true_residual_is_there_when_the_solve_returns(tmp_path):
+    """A host-side preconditioner leaves no sweep to check, so the residual's
+    copy is all that a solve still has to wait for."""
+    r = subprocess.run([str(build_host_precon(tmp_path))], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.stdout, r.stderr)
+    pairs = [[float(v) for v in line.split()[1:]] for line in r.stdout.splitlines()]
+    # r = b - A x in another order of summation: rounding of sums of 5 terms of order 1
+    assert len(pairs) == 2 and all(abs(d - h) <= 1e-12 + 1e-6 * h for d, h in pairs), pairs
