@@ -2384,7 +2384,11 @@ namespace lljbash {
 
 using pilu::DevBuf;
 
+// An apply is asynchronous: the solver's end waits for it, as freeing its
+// buffers did before they went to the pool, so that the caller may then reuse
+// the apply's vectors from any stream.
 IluSolver::~IluSolver() {
+    if (ext_ && ext_->n > 0 && hipDeviceSynchronize() != hipSuccess) (void)hipGetLastError();
     delete ext_;
     ext_ = nullptr;
     DestroyCsrMatrix(&aMatrix_);

@@ -121,3 +121,28 @@ def test_freed_blocks_are_reused_safely_and_given_back():
     assert not bad
     gc.collect()
     assert before - torch.cuda.mem_get_info()[0] < 64 << 20
+
+
+def test_destroying_a_solver_waits_for_its_applies():
+    """The vectors of an apply may be reused once its solver is gone, also while
+    other solvers live and keep the freed blocks in the pool."""
+    import torch
+
+    a = gen.poisson2d(300)
+    pair = []
+    for _ in range(2):
+        ilu = P.IluSolver(0)
+        ilu.SetMatrix(a.row_ptr, a.col_idx, a.value)
+        assert ilu.SetupMatrix() == 0 and ilu.Factorize() == 0
+        ilu.SetSweepMode(0, 0, 0)
+        pair.append(ilu)
+    b = torch.ones(a.n, dtype=torch.float64, device="cuda")
+    x = torch.zeros_like(b)
+    torch.cuda.synchronize()
+    done = torch.cuda.Event()
+    for _ in range(50):  # about 1.3 ms each
+        pair[0].SubstituteDevice(b.data_ptr(), x.data_ptr())
+    done.record()
+    under_way = not done.query()
+    pair[0].close()
+    assert under_way and done.query()
