@@ -67,28 +67,31 @@ public:
     void* take(size_t bytes) {
         int dev = 0;
         PILU_HIP(hipGetDevice(&dev));
-        std::lock_guard<std::mutex> lock(mu_);
+        std::unique_lock<std::mutex> lock(mu_);
         size_t at = free_.size();
         for (size_t i = 0; i < free_.size(); ++i) {
             const Block& f = free_[i];
             if (f.dev == dev && f.bytes >= bytes && f.bytes - bytes <= bytes / 4 && (at == free_.size() || f.bytes < free_[at].bytes))
                 at = i;
         }
-        if (at < free_.size() && free_[at].dirty) {
-            if (hipDeviceSynchronize() == hipSuccess) {
-                for (Block& f : free_)
-                    if (f.dev == dev) f.dirty = false;
-            } else {  // for instance while a stream is captured
-                (void)hipGetLastError();
-                at = free_.size();
-            }
-        }
         if (at < free_.size()) {
-            const Block f = free_[at];
-            used_.emplace(f.p, f);
+            Block f = free_[at];
+            used_.emplace(f.p, f);  // nobody else's from here on
             free_.erase(free_.begin() + static_cast<long>(at));
             held_ -= f.bytes;
-            return f.p;
+            if (!f.dirty) return f.p;
+            const long given = given_;
+            lock.unlock();  // other threads need not wait for what this one waits for
+            const bool idle = hipDeviceSynchronize() == hipSuccess;
+            if (!idle) (void)hipGetLastError();  // for instance while a stream is captured
+            lock.lock();
+            if (idle) {
+                for (Block& q : free_)
+                    if (q.dev == dev && q.given <= given) q.dirty = false;
+                return f.p;
+            }
+            used_.erase(f.p);
+            put_back(f);
         }
         void* p = nullptr;
         hipError_t rc = hipMalloc(&p, bytes);
@@ -99,7 +102,7 @@ public:
         }
         PILU_HIP(rc);
         try {
-            used_.emplace(p, Block{p, bytes, dev, false});
+            used_.emplace(p, Block{p, bytes, dev, false, 0});
         } catch (...) {
             (void)hipFree(p);
             throw;
@@ -116,13 +119,9 @@ public:
         }
         Block f = it->second;
         f.dirty = true;
+        f.given = ++given_;
         used_.erase(it);
-        try {
-            free_.push_back(f);
-            held_ += f.bytes;
-        } catch (...) {
-            (void)hipFree(p);
-        }
+        put_back(f);
         trim(used_.empty() ? 0 : kPoolBytes);
     }
 
@@ -132,7 +131,17 @@ private:
         size_t bytes;
         int dev;
         bool dirty;  // freed since the device was last waited for
+        long given;  // number of the free it came with
     };
+
+    void put_back(const Block& f) noexcept {
+        try {
+            free_.push_back(f);
+            held_ += f.bytes;
+        } catch (...) {
+            (void)hipFree(f.p);
+        }
+    }
 
     void trim(size_t keep) {
         size_t n = 0;
@@ -147,6 +156,7 @@ private:
     std::unordered_map<void*, Block> used_;
     std::vector<Block> free_;  // oldest first
     size_t held_ = 0;
+    long given_ = 0;
 };
 
 // Never destroyed: solvers with static storage are freed through it at exit.

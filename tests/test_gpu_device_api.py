@@ -146,3 +146,44 @@ def test_destroying_a_solver_waits_for_its_applies():
     under_way = not done.query()
     pair[0].close()
     assert under_way and done.query()
+
+
+def test_an_allocation_that_waits_does_not_hold_up_other_threads():
+    """A thread that takes a freed block waits for the device; another one whose
+    allocations find no freed block is through before the device is idle."""
+    import threading
+    import time
+
+    import torch
+
+    from par_ilu0_cpp_amd.learned import Gnn
+
+    a = gen.poisson2d(250)
+
+    def build():
+        ilu = P.IluSolver(0)
+        ilu.SetMatrix(a.row_ptr, a.col_idx, a.value)
+        assert ilu.SetupMatrix() == 0
+        return ilu
+
+    Gnn()  # its kernels are loaded
+    keep, gone = build(), build()
+    gone.close()
+    m = torch.rand(8192, 8192, device="cuda")
+    side, done = torch.cuda.Stream(), torch.cuda.Event()
+    with torch.cuda.stream(side):
+        torch.mm(m, m)
+        torch.cuda.synchronize()
+        for _ in range(150):
+            torch.mm(m, m)
+        done.record()
+    built = []
+    waiting = threading.Thread(target=lambda: built.append(build()))
+    waiting.start()
+    time.sleep(0.1)
+    assert waiting.is_alive() and not done.query()
+    net = Gnn()
+    through = not done.query()
+    waiting.join()
+    torch.cuda.synchronize()
+    assert through and len(built) == 1 and net is not None and keep is not None
