@@ -474,11 +474,14 @@ __device__ __forceinline__ void b_gate(BCtl& q, int i) {
 //
 // Workgroups take the chunks of `list` in order through tickets; a system's
 // chunks have consecutive tickets.  So only the newest system can be partly
-// started, and the launch drains as long as its chunks fit beside each other
-// wherever the hardware puts them, in the worst case on one XCD of 32 CUs with
-// 4 workgroups each; half of that (kBmaChunks) leaves room for another solve
-// doing the same.  Larger systems take one launch per term.  Partial slots
-// come in two generations by step parity, each step re-arming the other one.
+// started, and the launch drains as long as its chunks fit beside each other.
+// A CU holds two workgroups (176 to 185 registers; 64 KiB of LDS at most), an XCD
+// of 32 CUs 64: kBmaChunks fit wherever the hardware puts them, and as it deals
+// workgroups to the eight XCDs in turn, several solves doing the same do.
+// fused_chunks() asks for the occupancy: where a device is a smaller partition,
+// twice the largest system's chunks have to fit.  Larger systems take one
+// launch per term.  Partial slots come in two generations by step parity, each
+// step re-arming the other one.
 //
 // One launch per term read v_j, v_j+1 and w and wrote w each time: 35 us per
 // term on 40 systems x 8 right-hand sides, 147 of a solve's 379 ms.
@@ -793,6 +796,7 @@ public:
         sc[nsys] = static_cast<int>(beg.size());
         nchunks_ = static_cast<int>(beg.size());
         nfused_ = static_cast<int>(list_f.size());
+        fused_m_ = -1;
         list_f.insert(list_f.end(), list_b.begin(), list_b.end());
         chunk_list_.resize(list_f.size());
         sys_big_.resize(big.size());
@@ -1140,9 +1144,25 @@ private:
 
     size_t mgs_lds(int m) const { return sizeof(double) * K_ * (static_cast<size_t>(max_nc_) + 3 * (m + 2)); }
 
-    // Chunks of k_bmgs_all (the first of chunk_list_): none where the
-    // rotations of a long restart exceed the LDS.
-    int fused_chunks(int m) const { return mgs_lds(m) <= 64 * 1024 ? nfused_ : 0; }
+    // Chunks of k_bmgs_all (the first of chunk_list_): none where the rotations
+    // of a long restart exceed the LDS, or where the device has no room for the
+    // largest system's chunks twice (for another solve doing the same).
+    int fused_chunks(int m) {
+        if (fused_m_ == m) return fused_;
+        fused_m_ = m;
+        fused_ = 0;
+        if (nfused_ == 0 || mgs_lds(m) > 64 * 1024) return 0;
+        const void* kern = K_ == 1   ? reinterpret_cast<const void*>(k_bmgs_all<1>)
+                           : K_ == 2 ? reinterpret_cast<const void*>(k_bmgs_all<2>)
+                           : K_ == 4 ? reinterpret_cast<const void*>(k_bmgs_all<4>)
+                                     : reinterpret_cast<const void*>(k_bmgs_all<8>);
+        int dev = 0, cus = 0, per_cu = 0;
+        PILU_HIP(hipGetDevice(&dev));
+        PILU_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        PILU_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kBThreads, mgs_lds(m)));
+        if (2L * max_nc_ <= static_cast<long>(cus) * per_cu) fused_ = nfused_;
+        return fused_;
+    }
 
     void mgs_all_launch(int i, int m, const double* v, double* w, long nk, const double* part0, long hstride, Ext* ie) {
         const uint64_t wd = watchdog_ticks(ie->watchdog_s);
@@ -1233,6 +1253,7 @@ private:
     // Gram-Schmidt: chunks of the systems k_bmgs_all takes come first in
     // chunk_list_; most chunks of one of them
     int nfused_ = 0, max_nc_ = 0;
+    int fused_m_ = -1, fused_ = 0;  // fused_chunks(fused_m_)
     DevBuf<int> chunk_list_, sys_big_, sys_all_;
     DevBuf<double> pbuf_;
     DevBuf<int> tick_;

@@ -195,3 +195,31 @@ def torch_dev(v):
     import torch
 
     return torch.from_numpy(np.ascontiguousarray(v)).cuda()
+
+
+@pytest.mark.parametrize("m", [200, 336, 337])
+def test_batched_long_restarts(oracle, m):
+    """Restarts whose rotations leave two workgroups of the one-launch
+    Gram-Schmidt on a CU, fill its 64 KiB of LDS (8 + 3 * 338 doubles per
+    right-hand side of 1024), and exceed them (one launch per term)."""
+    import torch
+
+    mats, nrhs, tol = make_batch([60, 9, 21], seed=m), 8, 1e-8
+    rp, ci, va, sp = P.block_diagonal(mats)
+    n = rp.size - 1
+    B = np.random.default_rng(m).uniform(-1, 1, size=(n, nrhs))
+    d_rp, d_ci, d_va, d_b = to_dev(rp, ci, va, B)
+    d_x = torch.zeros((n, nrhs), dtype=torch.float64, device="cuda")
+    bg = P.BatchGmres()
+    assert bg.Setup(n, d_rp.data_ptr(), d_ci.data_ptr(), 0, sp, nrhs) == ci.size
+    assert bg.Factorize(d_va.data_ptr()) == 0
+    _, its, conv, rel = bg.Solve(d_rp.data_ptr(), d_ci.data_ptr(), d_va.data_ptr(), d_b.data_ptr(), d_x.data_ptr(),
+                                 tol, m, 500)
+    assert conv.all() and np.all(rel <= 1.01 * tol)
+    for s, a in enumerate(mats):
+        fac, dg, _ = oracle.ilu_factorize(a.row_ptr, a.col_idx, a.value)
+        for r in range(nrhs):
+            b = B[sp[s]:sp[s + 1], r]
+            ok_o, its_o, _, _ = oracle.gmres((a.row_ptr, a.col_idx, a.value), b, tol * np.linalg.norm(b), m, 500,
+                                             factors=(a.row_ptr, a.col_idx, dg, fac))
+            assert ok_o and abs(int(its[s, r]) - its_o) <= 1, (s, r, its[s, r], its_o)
