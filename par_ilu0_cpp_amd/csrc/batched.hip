@@ -842,7 +842,8 @@ public:
 
     int solve(const CsrMatrix* d_a, const double* d_rhs, double* d_sol, double rel_tol, int m, int maxits, int* its,
               int* conv, double* rel) {
-        if (!ready_) throw std::runtime_error("batched: factorize first");
+        // another precision than the factors' asks for a new factorization
+        if (!ready_ || !ilu_.DeviceState()->factored) throw std::runtime_error("batched: factorize first");
         if (d_a->size != n_) throw std::runtime_error("batched: matrix size changed");
         PILU_HIP(hipDeviceSynchronize());  // caller's null-stream work is complete
         const int ni = nsys_ * K_;

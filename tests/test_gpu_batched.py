@@ -223,3 +223,24 @@ def test_batched_long_restarts(oracle, m):
             ok_o, its_o, _, _ = oracle.gmres((a.row_ptr, a.col_idx, a.value), b, tol * np.linalg.norm(b), m, 500,
                                              factors=(a.row_ptr, a.col_idx, dg, fac))
             assert ok_o and abs(int(its[s, r]) - its_o) <= 1, (s, r, its[s, r], its_o)
+
+
+def small_batch(nrhs):
+    mats = make_batch([9, 14], seed=2)
+    rp, ci, va, sp = P.block_diagonal(mats)
+    d = to_dev(rp, ci, va, np.ones((rp.size - 1, nrhs)), np.zeros((rp.size - 1, nrhs)))
+    return rp.size - 1, sp, d, lambda bg: bg.Solve(*[t.data_ptr() for t in d], 1e-8, 30, 200)
+
+
+def test_batched_precision_change_asks_for_a_factorization():
+    n, sp, d, solve = small_batch(2)
+    bg = P.BatchGmres()
+    assert bg.Setup(n, d[0].data_ptr(), d[1].data_ptr(), 0, sp, 2) > 0
+    assert bg.Factorize(d[2].data_ptr()) == 0
+    assert solve(bg)[2].all()
+    bg.SetFactorPrecision(32)
+    with pytest.raises(RuntimeError):
+        solve(bg)
+    assert bg.Factorize(d[2].data_ptr()) == 0
+    d[4].zero_()
+    assert solve(bg)[2].all()
