@@ -774,6 +774,7 @@ public:
         if (nsys <= 0 || sys_ptr[0] != 0 || sys_ptr[nsys] != d_a->size) throw std::runtime_error("bad sys_ptr");
         if (!stream_) PILU_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
         drop_graph();
+        ready_ = set_up_ = false;  // from here on nothing fits the old factors, also if this set-up fails
         K_ = nrhs;
         nsys_ = nsys;
         n_ = d_a->size;
@@ -825,11 +826,12 @@ public:
         block_level_schedule(ie, true, row_sys_.get(), nsys, sperm_u_, sgrp_u_, soff_u_);
         build_rounds(ie);
         PILU_HIP(hipDeviceSynchronize());
-        ready_ = false;
+        set_up_ = true;
         return nnz_f;
     }
 
     bool factorize(const double* d_avals) {
+        if (!set_up_) throw std::runtime_error("batched: set up first");
         PILU_HIP(hipDeviceSynchronize());
         const bool ok = ilu_.FactorizeDeviceFromA(d_avals);
         if (br_kp_ > 0) gather_rounds(ilu_.DeviceState());
@@ -1259,7 +1261,7 @@ private:
     DevBuf<double> pbuf_;
     DevBuf<int> tick_;
     int K_ = 8, nsys_ = 0, n_ = 0, nchunks_ = 0, m_ = -1, maxits_ = -1, cycles_ = 0;
-    bool ready_ = false;
+    bool set_up_ = false, ready_ = false;
     DevBuf<int> chunk_beg_, chunk_sys_, sys_chunk_, row_sys_, flags_, int_out_;
     DevBuf<int> sperm_l_, sgrp_l_, soff_l_, sperm_u_, sgrp_u_, soff_u_;  // per-system level schedules
     DevBuf<double> v_, z_, hh_, part_, y_, res_, dbl_out_;

@@ -244,3 +244,19 @@ def test_batched_precision_change_asks_for_a_factorization():
     assert bg.Factorize(d[2].data_ptr()) == 0
     d[4].zero_()
     assert solve(bg)[2].all()
+
+
+def test_batched_failed_setup_leaves_nothing_to_solve_with():
+    """A set-up that is refused (an empty system) has replaced the old one's
+    counts already: no factorization and no solve until one succeeds."""
+    n, sp, d, solve = small_batch(2)
+    bg = P.BatchGmres()
+    assert bg.Setup(n, d[0].data_ptr(), d[1].data_ptr(), 0, sp, 2) > 0
+    assert bg.Factorize(d[2].data_ptr()) == 0
+    assert bg.Setup(n, d[0].data_ptr(), d[1].data_ptr(), 0, [0, sp[1], sp[1], n], 2) < 0
+    assert bg.Factorize(d[2].data_ptr()) < 0
+    with pytest.raises(RuntimeError):
+        solve(bg)
+    assert bg.Setup(n, d[0].data_ptr(), d[1].data_ptr(), 0, sp, 2) > 0
+    assert bg.Factorize(d[2].data_ptr()) == 0
+    assert solve(bg)[2].all()
