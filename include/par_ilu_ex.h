@@ -134,7 +134,7 @@ int IluSolverFactorizeDeviceEx(IluSolverHdl hdl, const double* d_values, int val
  * pattern, in a GMRES solve or alone.  That one replaces the level-scheduled
  * sweeps by faster ones where the pattern suits them: it allocates device
  * memory (mostly one to three times the factors'), waits for the stream and
- * takes as long as one to three applies before.  Results keep their bits.
+ * takes as long as one to five of the applies before it.  Results keep their bits.
  * "default_sweeps" of IluSolverScheduleJsonEx tells the form in use ("level
  * rows", "one workgroup", "tiles", "level walk") and its bytes;
  * IluSolverSetSweepModeEx(hdl, 0, 0, 0) keeps the level-scheduled sweeps. */

@@ -366,7 +366,10 @@ __global__ __launch_bounds__(kMgsThreads) void k_mgs_all(int n, int i, int m, in
 
 // The same for n <= kSmallRows in one workgroup: every reduction stays in it,
 // where the grid's hand-offs cost 3.8 us per term (58 us per step on 2D Poisson
-// 64^2).  Basis vectors are requested two terms ahead.
+// 64^2).  Basis vectors are requested two terms ahead.  kSmallRows is what the
+// registers hold (eight rows a thread), still short of the crossing: a whole step
+// (sweeps and SpMV too) takes 76 us here and 122 by the grid at n = 4096, restart
+// 30; 96 and 135 at 6400; 107 and 144 at 8100, and 155 and 217 there at restart 100.
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallRows = 8 * kSmallThreads;
 

@@ -1133,7 +1133,9 @@ __device__ __forceinline__ void guard_pivot(const PivotGuard& pg, double* piv, i
 // applied; its columns are matched once, before its values are waited for.
 // Rows of 266 entries and 133 pivots (ILU(2) of a random band, n = 40k):
 // 28.2 -> 16.2 ms, with LDS for the longest row (788 entries: sixteen rows per
-// CU) instead of 2560 entries (four).
+// CU) instead of 2560 entries (four).  Two or four entries per lane ahead take the
+// same time (the solve 38.1 and 37.9 ms, with 4 and 6 steps ahead in its level
+// walks); eight, and eight steps, 42.5.
 // ---------------------------------------------------------------------
 constexpr int kFacAhead = 4;
 

@@ -38,7 +38,7 @@ using Ext = lljbash::IluSolver::Ext;
 namespace {
 
 constexpr int kWalkWaves = 8;
-constexpr int kWalkAhead = 6;      // most steps requested ahead (k_walk)
+constexpr int kWalkAhead = 6;      // most steps requested ahead (k_walk); see kFacAhead for 4 and 8
 constexpr int kWalkRing = 1 << 14;
 constexpr unsigned kWalkFar = 0x80000000u;  // in an entry's slot: a row, to be read from memory
 // step flags; the barriers before the step are counted above them
